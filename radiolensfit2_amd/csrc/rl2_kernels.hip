@@ -1074,8 +1074,138 @@ __device__ inline void block_allreduce(double (&v)[N], double *lds)
     __syncthreads();
 }
 
+// Sum of v over the 64 lanes of a wave, in lane 63, by data-parallel-primitive moves (VALU
+// lane shifts, no LDS round trips): shifts by 1, 2, 4 and 8 within each row of 16 lanes
+// leave each row's total in its lane 15; row_bcast:15 adds row 0's total into row 1 and
+// row 2's into row 3, row_bcast:31 adds lane 31's into rows 2 and 3.  Lanes whose source
+// lies outside the row or is masked off add 0.  A fixed order, so the sum is deterministic.
+template <int CTRL, int ROW_MASK, int BANK_MASK>
+__device__ inline double dpp_f64(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    const int rlo = __builtin_amdgcn_update_dpp(0, lo, CTRL, ROW_MASK, BANK_MASK, false);
+    const int rhi = __builtin_amdgcn_update_dpp(0, hi, CTRL, ROW_MASK, BANK_MASK, false);
+    return __hiloint2double(rhi, rlo);
+}
+__device__ inline double wave_sum_last(double v)
+{
+    v += dpp_f64<0x111, 0xf, 0xf>(v);  // row_shr:1
+    v += dpp_f64<0x112, 0xf, 0xf>(v);  // row_shr:2
+    v += dpp_f64<0x114, 0xf, 0xf>(v);  // row_shr:4
+    v += dpp_f64<0x118, 0xf, 0xf>(v);  // row_shr:8
+    v += dpp_f64<0x142, 0xa, 0xf>(v);  // row_bcast:15 into rows 1 and 3
+    v += dpp_f64<0x143, 0xc, 0xf>(v);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+// The wave's sum in every lane: wave_sum_last, then lane 63's value read into scalar
+// registers (every lane gets the same value, so the wave takes the same branches after it).
+__device__ inline double wave_sum(double v)
+{
+    v = wave_sum_last(v);
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
+    return __hiloint2double(hi, lo);
+}
+
+// Lane values read into scalar registers (l uniform over the wave).
+__device__ inline double read_lane(double v, int l)
+{
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+    return __hiloint2double(hi, lo);
+}
+
+// The wave's maximum (MAX) or minimum in every lane, by the lane shifts of wave_sum_last; a
+// lane whose source lies outside its row, or in a row masked off, keeps its own value, which
+// leaves the extreme unchanged.  fmax and fmin are exact (and skip NaN), so the result does
+// not depend on the order.
+template <int CTRL, int ROW_MASK>
+__device__ inline double dpp_keep_f64(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    const int rlo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROW_MASK, 0xf, false);
+    const int rhi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROW_MASK, 0xf, false);
+    return __hiloint2double(rhi, rlo);
+}
+template <bool MAX>
+__device__ inline double wave_extreme(double v)
+{
+    auto op = [](double p, double q) { return MAX ? fmax(p, q) : fmin(p, q); };
+    v = op(v, dpp_keep_f64<0x111, 0xf>(v));  // row_shr:1
+    v = op(v, dpp_keep_f64<0x112, 0xf>(v));  // row_shr:2
+    v = op(v, dpp_keep_f64<0x114, 0xf>(v));  // row_shr:4
+    v = op(v, dpp_keep_f64<0x118, 0xf>(v));  // row_shr:8
+    v = op(v, dpp_keep_f64<0x142, 0xa>(v));  // row_bcast:15 into rows 1 and 3
+    v = op(v, dpp_keep_f64<0x143, 0xc>(v));  // row_bcast:31 into rows 2 and 3
+    return read_lane(v, 63);
+}
+
+// The wave's inclusive prefix products, by the lane shifts of wave_sum_last; a lane without a
+// source keeps its own value (times 1).
+template <int CTRL, int ROW_MASK>
+__device__ inline double dpp_one_f64(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    const int rlo = __builtin_amdgcn_update_dpp(0, lo, CTRL, ROW_MASK, 0xf, false);
+    const int rhi = __builtin_amdgcn_update_dpp(0x3ff00000, hi, CTRL, ROW_MASK, 0xf, false);
+    return __hiloint2double(rhi, rlo);
+}
+__device__ inline double wave_scan_mul(double v)
+{
+    v *= dpp_one_f64<0x111, 0xf>(v);  // row_shr:1
+    v *= dpp_one_f64<0x112, 0xf>(v);  // row_shr:2
+    v *= dpp_one_f64<0x114, 0xf>(v);  // row_shr:4
+    v *= dpp_one_f64<0x118, 0xf>(v);  // row_shr:8
+    v *= dpp_one_f64<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    v *= dpp_one_f64<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+// expint_ei (rl2_math.h) by a wave, for an argument that is the same in all its lanes: lane k
+// takes the series' term k + 1.  The terms are prefix products of x / k (power series) or
+// k / x (asymptotic series, cut at its smallest term and at eps / 4), each of at most six
+// roundings where the recurrence takes 2 k, and 64 of them cost two divisions and twelve lane
+// shifts instead of a chain of 128 divisions.
+__device__ inline double expint_ei_wave(double x)
+{
+    const double euler = 0.57721566490153286060651209008240243;
+    constexpr double kQuarterEps = 2.220446049250313e-16 * 0.25;
+    const int lane = threadIdx.x & 63;
+    if (x <= 40.) {
+        double sum = 0., carry = 1.;
+        for (int b = 0; b < 16; b++) {
+            const double k = (double)(64 * b + lane + 1);
+            const double p = carry * wave_scan_mul(x / k);
+            const double t = p / k;
+            sum += wave_sum(t);
+            if (read_lane(t, 63) < kQuarterEps * sum) break;
+            carry = read_lane(p, 63);
+        }
+        return euler + log(x) + sum;
+    }
+    const double k = (double)(lane + 1);
+    const double t = wave_scan_mul(k / x);
+    const double sum = 1. + wave_sum(k < x && t >= kQuarterEps ? t : 0.);
+    return exp(x) / x * sum;
+}
+
+// marg_position (rl2_math.h) by a wave, for an argument that is the same in all its lanes.
+// The two exponential integrals were the longest serial chain of a task that ends with
+// B <= 100 (a hundred dependent divisions each, by one lane).
+__device__ inline double marg_position_wave(double x)
+{
+    const double Delta = 0.5 * 5.991;
+    if (x <= Delta) return kBad;
+    if (x > 100.) return x - log(Delta) - exp(-Delta);
+    if ((x - Delta) < 0.0001) x = Delta + 0.0001;
+    const double yc = expint_ei_wave(x), ys = expint_ei_wave(x - Delta);
+    return log((yc - ys) / log(x / (x - Delta)));
+}
+
 // likelihood.c:174-183: L_r = log of the position-marginalised likelihood minus
-// 1/2 log det of the cross-correlation Hessian; -1e10 when the peak search failed.
+// 1/2 log det of the cross-correlation Hessian; -1e10 when the peak search failed.  Called
+// by a whole wave with the same arguments in every lane; lane 0 writes.
 __device__ inline void finish_lr(const LikLaunch &a, int item, int r, double ho,
                                  double det_sigma, int iter)
 {
@@ -1084,12 +1214,13 @@ __device__ inline void finish_lr(const LikLaunch &a, int item, int r, double ho,
         L = kBad;
     else {
         const double B = (ho * ho) * 0.5;
-        L = marg_position(B);
+        L = marg_position_wave(B);
         if (isnan(L))
             L = kBad;
         else
             L -= 0.5 * log(det_sigma);
     }
+    if ((threadIdx.x & 63) != 0) return;
     a.Lr[(size_t)item * kMaxR + r] = L;
     a.nit[(size_t)item * kMaxR + r] = iter;
     if (a.ho) a.ho[(size_t)item * kMaxR + r] = ho;
@@ -1206,7 +1337,7 @@ __global__ __launch_bounds__(BS) void likelihood_kernel(LikLaunch a)
         det = dxx * dyy - dxy * dxy;
         norm = sqrt(incx * incx + incy * incy);
     }
-    if (tid == 0)
+    if (tid < 64)
         finish_lr(a, item, r, gmod ? value : value / sqrt(S2), gmod ? det : det / S2, iter);
 }
 
@@ -1364,7 +1495,7 @@ __global__ __launch_bounds__(BS) void likelihood32_kernel(LikLaunch a)
         det = dxx * dyy - dxy * dxy;
         norm = sqrt(incx * incx + incy * incy);
     }
-    if (tid == 0) finish_lr(a, item, r, value / sqrt(S2), det / S2, iter);
+    if (tid < 64) finish_lr(a, item, r, value / sqrt(S2), det / S2, iter);
 }
 
 void launch_likelihood(hipStream_t s, const LikLaunch &a)
@@ -1665,73 +1796,6 @@ __device__ double marginalise_posterior(int num, const double *x, double *y, Qag
 // 63's, read into scalar registers), so all lanes follow the same control flow.  The sums
 // differ from QUADPACK's sequential order only by rounding.  Each bisection integrates its
 // two halves on the two waves at once.
-
-// Sum of v over the 64 lanes of a wave, in lane 63, by data-parallel-primitive moves (VALU
-// lane shifts, no LDS round trips): shifts by 1, 2, 4 and 8 within each row of 16 lanes
-// leave each row's total in its lane 15; row_bcast:15 adds row 0's total into row 1 and
-// row 2's into row 3, row_bcast:31 adds lane 31's into rows 2 and 3.  Lanes whose source
-// lies outside the row or is masked off add 0.  A fixed order, so the sum is deterministic.
-template <int CTRL, int ROW_MASK, int BANK_MASK>
-__device__ inline double dpp_f64(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    const int rlo = __builtin_amdgcn_update_dpp(0, lo, CTRL, ROW_MASK, BANK_MASK, false);
-    const int rhi = __builtin_amdgcn_update_dpp(0, hi, CTRL, ROW_MASK, BANK_MASK, false);
-    return __hiloint2double(rhi, rlo);
-}
-__device__ inline double wave_sum_last(double v)
-{
-    v += dpp_f64<0x111, 0xf, 0xf>(v);  // row_shr:1
-    v += dpp_f64<0x112, 0xf, 0xf>(v);  // row_shr:2
-    v += dpp_f64<0x114, 0xf, 0xf>(v);  // row_shr:4
-    v += dpp_f64<0x118, 0xf, 0xf>(v);  // row_shr:8
-    v += dpp_f64<0x142, 0xa, 0xf>(v);  // row_bcast:15 into rows 1 and 3
-    v += dpp_f64<0x143, 0xc, 0xf>(v);  // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
-// The wave's sum in every lane: wave_sum_last, then lane 63's value read into scalar
-// registers (every lane gets the same value, so the wave takes the same branches after it).
-__device__ inline double wave_sum(double v)
-{
-    v = wave_sum_last(v);
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
-    return __hiloint2double(hi, lo);
-}
-
-// Lane values read into scalar registers (l uniform over the wave).
-__device__ inline double read_lane(double v, int l)
-{
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
-}
-
-// The wave's maximum (MAX) or minimum in every lane, by the lane shifts of wave_sum_last; a
-// lane whose source lies outside its row, or in a row masked off, keeps its own value, which
-// leaves the extreme unchanged.  fmax and fmin are exact (and skip NaN), so the result does
-// not depend on the order.
-template <int CTRL, int ROW_MASK>
-__device__ inline double dpp_keep_f64(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    const int rlo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROW_MASK, 0xf, false);
-    const int rhi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROW_MASK, 0xf, false);
-    return __hiloint2double(rhi, rlo);
-}
-template <bool MAX>
-__device__ inline double wave_extreme(double v)
-{
-    auto op = [](double p, double q) { return MAX ? fmax(p, q) : fmin(p, q); };
-    v = op(v, dpp_keep_f64<0x111, 0xf>(v));  // row_shr:1
-    v = op(v, dpp_keep_f64<0x112, 0xf>(v));  // row_shr:2
-    v = op(v, dpp_keep_f64<0x114, 0xf>(v));  // row_shr:4
-    v = op(v, dpp_keep_f64<0x118, 0xf>(v));  // row_shr:8
-    v = op(v, dpp_keep_f64<0x142, 0xa>(v));  // row_bcast:15 into rows 1 and 3
-    v = op(v, dpp_keep_f64<0x143, 0xc>(v));  // row_bcast:31 into rows 2 and 3
-    return read_lane(v, 63);
-}
 
 // The spline of the r-marginalisation in LDS with the cubic coefficients b_i and d_i of each
 // interval (cspline_eval's), formed once per spline: spline_exp_lds then takes no division
@@ -2770,19 +2834,30 @@ __device__ int newton_update(TileTask &T, const double (&v)[7], double *ho_out,
     return 1;
 }
 
+// finish_lr of a step that a whole wave took, when lane 63, which holds the task's totals,
+// ended the task: its values go to every lane for the wave-parallel position marginalisation.
+__device__ inline void finish_lane63(const LikLaunch &a, int item, int r, int done, double ho,
+                                     double det, int iter)
+{
+    if (__builtin_amdgcn_readlane(done, 63))
+        finish_lr(a, item, r, read_lane(ho, 63), read_lane(det, 63),
+                  __builtin_amdgcn_readlane(iter, 63));
+}
+
 // newton_update on the task's state in memory, writing L_r when the task finishes (the
 // step kernel of the two-kernel passes).
 // The state is read from T and written to To (the same task in another buffer when the
-// passes keep two generations of state; T itself otherwise).
+// passes keep two generations of state; T itself otherwise).  Called by a whole wave whose
+// lane 63 holds the sums; that lane writes the state, and its return value and offset count.
 template <int PASS>
 __device__ int tile_step(const LikLaunch &a, const TileTask *T, TileTask *To, int item, int r,
                          const double (&v)[7], double *xo, double *yo)
 {
     TileTask S = *T;
-    double ho, det;
+    double ho = 0., det = 0.;
     const int done = newton_update<PASS>(S, v, &ho, &det);
-    *To = S;
-    if (done) finish_lr(a, item, r, ho, det, S.iter);
+    if ((threadIdx.x & 63) == 63) *To = S;
+    finish_lane63(a, item, r, done, ho, det, S.iter);
     *xo = S.xo;
     *yo = S.yo;
     return done;
@@ -3063,7 +3138,12 @@ __global__ __launch_bounds__(kStepBS) void lik_step_kernel(TileLaunch t)
             double v[7];
             task_sums(t.partials + (size_t)(first + (unsigned)(r - t.r_lo)) * 8, nch, nr, lane,
                       v);
-            if (lane == 63) go = !tile_step<PASS>(a, T, To, item, r, v, &s_off[0], &s_off[1]);
+            double xo, yo;
+            go = !tile_step<PASS>(a, T, To, item, r, v, &xo, &yo);
+            if (lane == 63) {
+                s_off[0] = xo;
+                s_off[1] = yo;
+            }
         } else if (lane == 63 && To != T) {
             *To = *T;  // a finished task keeps its state in the other generation too
         }
@@ -3159,11 +3239,9 @@ __device__ __attribute__((always_inline)) inline void fused_step(const TileLaunc
     int go = 0;
     double xo = 0., yo = 0.;
     if (t.mode == 2) {
-        if (lane == 63) {
-            go = pre.S.active;
-            xo = pre.S.xo;
-            yo = pre.S.yo;
-        }
+        go = pre.S.active;
+        xo = pre.S.xo;
+        yo = pre.S.yo;
     } else {
         double v[7];
         if (nch <= 64) {  // task_sums' arithmetic on the chunk sums read at the start
@@ -3180,19 +3258,18 @@ __device__ __attribute__((always_inline)) inline void fused_step(const TileLaunc
             task_sums(t.part_in + (size_t)(first + (unsigned)(r - t.r_lo)) * 8, nch, t.nr_g,
                       lane, v);
         }
-        if (lane == 63) {
-            TileTask S = t.mode == 0 ? TileTask{} : pre.S;
-            double ho, det;
-            const int done = t.mode == 0 ? newton_update<0>(S, v, &ho, &det)
-                                         : newton_update<1>(S, v, &ho, &det);
-            if (chunk == 0) {
-                t.tasks_out[ti] = S;
-                if (done) finish_lr(a, item, r, ho, det, S.iter);
-            }
-            go = !done;
-            xo = S.xo;
-            yo = S.yo;
+        // the totals, and so the step, are lane 63's: the other lanes take it on partial sums
+        TileTask S = t.mode == 0 ? TileTask{} : pre.S;
+        double ho = 0., det = 0.;
+        const int done = t.mode == 0 ? newton_update<0>(S, v, &ho, &det)
+                                     : newton_update<1>(S, v, &ho, &det);
+        if (chunk == 0) {
+            if (lane == 63) t.tasks_out[ti] = S;
+            finish_lane63(a, item, r, done, ho, det, S.iter);
         }
+        go = !done;
+        xo = S.xo;
+        yo = S.yo;
     }
     if (lane == 63) {
         *go_out = go;
@@ -3372,7 +3449,7 @@ __device__ inline void task_sums_published(const double *P0, unsigned nch, int n
             v[j] += __hip_atomic_load(P0 + (size_t)c * nr * 8 + j, __ATOMIC_RELAXED,
                                       __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-    for (int j = 0; j < 7; j++) v[j] = wave_sum_last(v[j]);
+    for (int j = 0; j < 7; j++) v[j] = wave_sum_last(v[j]);  // totals in lane 63
 }
 
 // One block's share of an evaluation: a task, and the run of its chunks the block sums.
@@ -3495,20 +3572,18 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_persist_kernel(Pe
                     task_sums_published(p.part + ((size_t)(pass - 1) * t.nwg + K.first +
                                                   (unsigned)(K.r - 1)) * 8,
                                         K.nch, nr, lane, v);
+                    TileTask S = pass == 1 ? TileTask{} : K.S;
+                    double ho = 0., det = 0.;
+                    const int done = pass == 1 ? newton_update<0>(S, v, &ho, &det)
+                                               : newton_update<1>(S, v, &ho, &det);
                     if (lane == 63) {
-                        TileTask S = pass == 1 ? TileTask{} : K.S;
-                        double ho, det;
-                        const int done = pass == 1 ? newton_update<0>(S, v, &ho, &det)
-                                                   : newton_update<1>(S, v, &ho, &det);
                         K.S = S;
                         K.active = !done;
-                        if (done && K.c0 == 0) {
-                            p.t.tasks[ti] = S;
-                            finish_lr(a, K.item, K.r, ho, det, S.iter);
-                        }
+                        if (done && K.c0 == 0) p.t.tasks[ti] = S;
                         s_off[0] = S.xo;
                         s_off[1] = S.yo;
                     }
+                    if (K.c0 == 0) finish_lane63(a, K.item, K.r, done, ho, det, S.iter);
                 }
                 __syncthreads();
                 if (!K.active) continue;
@@ -3914,18 +3989,20 @@ void launch_marginalise_r(hipStream_t s, int num, const double *x, const double 
     marginalise_r_kernel<<<1, 1, 0, s>>>(num, x, y, out, qag_ws, qag_iws);
 }
 
-// marg_position (likelihood.c:376-421) on n given arguments, one per thread: the device
+// marg_position (likelihood.c:376-421) on n given arguments, one per wave: the device
 // function finish_lr applies to B = ho^2 / 2.
-__global__ void marg_position_kernel(int n, const double *x, double *out)
+__global__ __launch_bounds__(256) void marg_position_kernel(int n, const double *x, double *out)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = marg_position(x[i]);
+    const int i = blockIdx.x * (256 / 64) + (threadIdx.x >> 6);
+    if (i >= n) return;  // a whole wave
+    const double y = marg_position_wave(x[i]);
+    if ((threadIdx.x & 63) == 0) out[i] = y;
 }
 
 void launch_marg_position(hipStream_t s, int n, const double *x, double *out)
 {
     if (n <= 0) return;
-    marg_position_kernel<<<(n + 255) / 256, 256, 0, s>>>(n, x, out);
+    marg_position_kernel<<<(n + 3) / 4, 256, 0, s>>>(n, x, out);
 }
 
 // ------------------------------------------------------------------ subtraction (K2)
