@@ -331,6 +331,10 @@ struct TileLaunch {
                                // (0: they differ; the kernels then search chunk_first)
 };
 void launch_tile_pass(hipStream_t s, const TileLaunch &t, int pass);
+// Every pass of every task in one launch: items of at most kTaskChunks chunks of
+// kTileMinCells cells (chunks: the largest), on grid facets with records.
+constexpr unsigned kTaskChunks = 4;
+void launch_lik_task(hipStream_t s, const TileLaunch &t, unsigned chunks);
 // One Newton pass with the previous pass's step folded in (grid items, row tables in LDS).
 void launch_tile_fused(hipStream_t s, const TileLaunch &t);
 // Work-groups are dispatched to the 8 XCDs round-robin (block b to XCD b % 8), and each XCD

@@ -3629,6 +3629,208 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_persist_kernel(Pe
     }
 }
 
+// ------------------------------------------------------------------ small facets: one launch
+// The whole Newton search of one (item, r) task in one work-group, for facets of at most
+// kTaskChunks chunks of kTileMinCells cells with records (up to kRecFacet columns).  Such a
+// pass is latency: a launch per pass took 5 to 8 us, of which the cells are a few hundred
+// nanoseconds; here a pass is three barriers, and what is left of it is the chain of sums,
+// step, tables and cells.  Each group of 256 threads holds the cells of its NC chunks in
+// registers: D M (the model M does not depend on the offset) and the record offsets, so a
+// Newton pass reads only the records in LDS.  The chunks, a thread's cells and their order,
+// the chunk sums, the step and the table entries are those of pass 0 and the fused passes, so
+// every L_r is the same bit for bit by either route.
+// G groups of 256 threads; a task has at most G * NC chunks (chunk c: group c % G).
+// Measured against the passes: one point on 138 cells 64.1 -> 46.5 us, the loop over 24
+// galaxies of 175 to 2111 cells 38.5 -> 26.3 ms, in batches of 16 (48 galaxies) 18.4 -> 15.1
+// ms.  On 6,582 cells 1, 4 and 24 points took 69, 71 and 102 us by the passes and 60, 60 and
+// 96 here; from 8,192 cells on (twice the cells in registers, which spill) 71, 77 and 128
+// against 75, 76 and 139, so kTaskChunks is 4.
+template <int KIND, int G, int NC>
+__global__ __launch_bounds__(kTileBS *G) void lik_task_kernel(TileLaunch t)
+{
+    constexpr int BS = kTileBS * G, Q = kTileMinCells / kTileBS, W = kTileBS / 64;
+    constexpr int NJ = 7;
+    __shared__ double red[G * NC][W][NJ];
+    __shared__ TabRot<kRecFacet / kTabRun> R;
+    extern __shared__ double2 tab_lds[];  // t.tab_lds_facet records
+    RecEntry *rec = reinterpret_cast<RecEntry *>(tab_lds);
+    const char *recb = reinterpret_cast<const char *>(tab_lds);
+    if (KIND == 2 && blockIdx.x == 0 && threadIdx.x < t.n_inl)
+        t.items_w[threadIdx.x] = t.inl[threadIdx.x];
+    const LikLaunch &a = t.lk;
+    const int item = (int)(blockIdx.x / (unsigned)t.nr_g);
+    const int r = (int)(blockIdx.x - (unsigned)item * (unsigned)t.nr_g) + t.r_lo;
+    const LikItem it = (KIND == 2 ? t.inl : a.items)[item];
+    const FacetDev &F = a.facets[it.slot];
+    const unsigned n = F.n, gf = F.grid_facet;
+    const uint32_t *loff = F.loff;
+    const double2 *dc = F.dc;
+    const double *w2 = F.invs2_64, *ctr = F.ctr;
+    const unsigned nch = max(1u, (n + kTileMinCells - 1) / kTileMinCells);
+    const int g = threadIdx.x / kTileBS, lt = threadIdx.x % kTileBS;
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x / 64) % W;
+    // rows of 256 cells of the group's chunk k that hold any cell (uniform over the group)
+    auto rows = [&](int k) {
+        const unsigned beg = (unsigned)(g + k * G) * kTileMinCells;
+        return beg < n ? min((unsigned)Q, (n - beg + kTileBS - 1) / kTileBS) : 0u;
+    };
+    // the thread's cells: offsets and data, then D M (past the end: the zero pad cell n)
+    uint32_t o[NC][Q];
+    double hr[NC][Q], hi[NC][Q], s2[NC][Q];
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+        const unsigned nq = rows(k);
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            if ((unsigned)q >= nq) break;
+            const unsigned i =
+                min(n, (unsigned)(g + k * G) * kTileMinCells + q * kTileBS + (unsigned)lt);
+            o[k][q] = gload(loff, i);
+            const double2 d = gload(dc, i);
+            hr[k][q] = d.x;
+            hi[k][q] = d.y;
+            s2[k][q] = gload(w2, i);
+        }
+    }
+    for (unsigned k = threadIdx.x; k < gf; k += BS) rec[k].c = gload(ctr, k);
+    __syncthreads();
+    const double e1 = it.e1, e2 = it.e2;
+    const double detA = 1. - e1 * e1 - e2 * e2;
+    const double scale = arcs2rad_scale(a.rg.ro[r]);
+    const double sf = (scale * scale) / (detA * detA);
+    const double sw = sf * (4 * kPi * kPi);
+    const double a1 = 1. + e1, a2 = 1. - e1;
+    constexpr double kTwoPi2 = kTwoPi * kTwoPi;
+    // a chunk's sums of this wave, from lane 63
+    auto put = [&](int k, double (&s)[NJ], int nj) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+            if (j < nj) s[j] = wave_sum_last(s[j]);
+        if (lane == 63)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                if (j < nj) red[g + k * G][wave][j] = s[j];
+    };
+#pragma unroll
+    for (int k = 0; k < NC; k++) {  // pass 0: tile_sums64_p0_db's terms
+        double s[NJ] = {};
+        const unsigned nq = rows(k);
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            if ((unsigned)q >= nq) break;
+            const double uu = reinterpret_cast<const RecEntry *>(recb + (o[k][q] & 0xffffu))->c;
+            const double vv = reinterpret_cast<const RecEntry *>(recb + (o[k][q] >> 16))->c;
+            const double k1 = fma(e2, vv, a1 * uu);
+            const double k2 = fma(a2, vv, e2 * uu);
+            const double rr = rsqrt_ge1(fma(sw, fma(k1, k1, k2 * k2), 1.));
+            const double M = rr * rr * rr;
+            const double dr = hr[k][q], di = hi[k][q];
+            hr[k][q] = dr * M;
+            hi[k][q] = -di * M;
+            s[0] = fma(M * M, s2[k][q], s[0]);
+            s[1] += hr[k][q];
+            s[2] = fma(-hi[k][q], uu, s[2]);
+            s[3] = fma(-hi[k][q], vv, s[3]);
+            const double hU = hr[k][q] * uu;
+            s[4] = fma(-hU, uu, s[4]);
+            s[5] = fma(-hr[k][q] * vv, vv, s[5]);
+            s[6] = fma(-hU, vv, s[6]);
+        }
+        s[2] *= kTwoPi;
+        s[3] *= kTwoPi;
+        s[4] *= kTwoPi2;
+        s[5] *= kTwoPi2;
+        s[6] *= kTwoPi2;
+        put(k, s, 7);
+    }
+    TileTask S = {};
+    for (int pass = 0;; pass++) {
+        __syncthreads();
+        // every wave adds the task's chunk sums (tile_reduce's order over the waves, then
+        // task_sums' over the chunks) and takes the step from lane 63's totals
+        double v[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            double p = 0.;
+            if (lane < (int)nch) {
+#pragma unroll
+                for (int w = 0; w < W; w++) p += red[lane < G * NC ? lane : 0][w][j];
+            }
+            v[j] = 0.;
+            v[j] += p;
+            v[j] = wave_sum_last(v[j]);
+        }
+        double ho = 0., det = 0.;
+        const int done = pass == 0 ? newton_update<0>(S, v, &ho, &det)
+                                   : newton_update<1>(S, v, &ho, &det);
+        if (__builtin_amdgcn_readlane(done, 63)) {  // the same in every wave
+            if (threadIdx.x < 64) finish_lane63(a, item, r, done, ho, det, S.iter);
+            return;
+        }
+        const double xo = read_lane(S.xo, 63), yo = read_lane(S.yo, 63);
+        tab_rot_stage(R, RecCtr{rec}, gf, xo, yo, 0u, (gf + kTabRun - 1) / kTabRun - 1, false);
+        __syncthreads();
+        for (unsigned q = threadIdx.x; q < 2 * gf; q += BS) {
+            const unsigned k = q < gf ? q : q - gf;
+            const double2 e = q < gf ? tab_x(R, k) : tab_y(R, k);
+            double *d = q < gf ? &rec[k].xr : &rec[k].yr;
+            d[0] = e.x;
+            d[1] = e.y;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NC; k++) {  // tile_sums64_rec's terms
+            double s[NJ] = {};
+            const unsigned nq = rows(k);
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                if ((unsigned)q >= nq) break;
+                const RecEntry &col =
+                    *reinterpret_cast<const RecEntry *>(recb + (o[k][q] & 0xffffu));
+                const RecEntry &row = *reinterpret_cast<const RecEntry *>(recb + (o[k][q] >> 16));
+                const double uu = col.c, vv = row.c;
+                const double cs = fma(col.xr, row.yr, -(col.xi * row.yi));
+                const double sn = fma(col.xi, row.yr, col.xr * row.yi);
+                const double re = fma(hr[k][q], cs, -hi[k][q] * sn);
+                const double im = fma(hr[k][q], sn, hi[k][q] * cs);
+                s[0] += re;
+                s[1] = fma(-im, uu, s[1]);
+                s[2] = fma(-im, vv, s[2]);
+                const double rU = re * uu;
+                s[3] = fma(-rU, uu, s[3]);
+                s[4] = fma(-re * vv, vv, s[4]);
+                s[5] = fma(-rU, vv, s[5]);
+            }
+            s[1] *= kTwoPi;
+            s[2] *= kTwoPi;
+            s[3] *= kTwoPi2;
+            s[4] *= kTwoPi2;
+            s[5] *= kTwoPi2;
+            put(k, s, 6);
+        }
+    }
+}
+
+template <int KIND>
+static void launch_task_kind(hipStream_t s, const TileLaunch &t, unsigned chunks)
+{
+    const unsigned g = (unsigned)t.lk.nitems * (unsigned)t.nr_g, lds = t.tab_lds_facet * kRecBytes;
+    if (chunks <= 1)
+        lik_task_kernel<KIND, 1, 1><<<g, kTileBS, lds, s>>>(t);
+    else if (chunks <= 2)
+        lik_task_kernel<KIND, 2, 1><<<g, 2 * kTileBS, lds, s>>>(t);
+    else
+        lik_task_kernel<KIND, 2, 2><<<g, 2 * kTileBS, lds, s>>>(t);
+}
+
+void launch_lik_task(hipStream_t s, const TileLaunch &t, unsigned chunks)
+{
+    if (t.grid == 2)
+        launch_task_kind<2>(s, t, chunks);
+    else
+        launch_task_kind<1>(s, t, chunks);
+}
+
 // Largest block count of a cooperative persistent launch with `lds` bytes of dynamic LDS
 // (0: the kernel cannot run).
 unsigned persist_capacity(unsigned lds, int kind)

@@ -750,7 +750,7 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
     bool tiled = o.lik_block == 0;
     for (int i = 0; i < n && tiled; i++)
         if (o.h_facets[items[i].slot].mod) tiled = false;  // given model: one group per (e, r)
-    const bool want_detail = Lr || nit || (g_stats_on && !tiled);
+    bool want_detail = Lr || nit || (g_stats_on && !tiled);
     // Every copy, fill and stream dependency queued below ANDs its status into q_ok, which
     // is checked with the launches' before the results are read.
     bool q_ok = true;
@@ -764,6 +764,22 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
                                          hipMemcpyDeviceToHost, g_stream),
                           "step count copy") &&
                    q_ok;
+    };
+    // FLOP-equivalents from the step counts: n * (37 + 25 N_it) per (item, r)
+    auto count_flops = [&]() {
+        double fl = 0.;
+        for (int i = 0; i < n; i++) {
+            const double nn = o.slots[items[i].slot].n;
+            for (int r = 1; r < o.rg.numr; r++)
+                fl += nn * (37. + 25. * b.h_nit[(size_t)i * kMaxR + r]);
+        }
+        stats_add_work(RL2_K_LIKELIHOOD, fl, 0.);
+    };
+    auto give = [&](double *Le, int *err, double *Lr, int *nit) {
+        memcpy(Le, b.h_Le, n * sizeof(double));
+        memcpy(err, b.h_err, n * sizeof(int));
+        if (Lr) memcpy(Lr, b.h_Lr, (size_t)n * kMaxR * sizeof(double));
+        if (nit) memcpy(nit, b.h_nit, (size_t)n * kMaxR * sizeof(int));
     };
     if (tiled) {
         // chunks per (item, r) from the host copy of each slot's cell count.  An item's chunk
@@ -788,13 +804,17 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
             }
             return chunk;
         };
-        unsigned chunks = 0;
+        unsigned chunks = 0, most_chunks = 0;
+        bool min_chunks = true;  // every item in the smallest chunks
         for (int i = 0; i < n; i++) {
             const unsigned cells = o.slots[items[i].slot].n;
             const unsigned chunk = item_chunk(cells, items[i].prec);
+            const unsigned nc = std::max(1u, (cells + chunk - 1) / chunk);
             b.h_items[i].chunk_first = chunks;
             b.h_items[i].chunk_cells = chunk;
-            chunks += std::max(1u, (cells + chunk - 1) / chunk);
+            chunks += nc;
+            most_chunks = std::max(most_chunks, nc);
+            min_chunks = min_chunks && chunk == kTileMinCells;
         }
         const unsigned total = chunks * (unsigned)nr;
         if (!b.ensure_partials(2 * (size_t)total)) return false;  // two generations
@@ -953,12 +973,32 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
                     return false;
                 }
                 if (g_stats_on) stats_add_work(RL2_K_LIKELIHOOD, *b.h_flops, 0.);
-                memcpy(Le, b.h_Le, n * sizeof(double));
-                memcpy(err, b.h_err, n * sizeof(int));
-                if (Lr) memcpy(Lr, b.h_Lr, (size_t)n * kMaxR * sizeof(double));
-                if (nit) memcpy(nit, b.h_nit, (size_t)n * kMaxR * sizeof(int));
+                give(Le, err, Lr, nit);
                 return true;
             }
+        }
+        // Small facets: every pass of a task in one work-group, one launch per evaluation,
+        // with the same bits as the passes.  A knob that shapes the passes keeps them.
+        if (fused && tuning().fuse_step == 1 && tg[0].tab_y_lds && min_chunks &&
+            most_chunks <= kTaskChunks && !tuning().tile_passes && !tuning().tile_blocks &&
+            !tuning().tile_cells && tuning().p0_tasks == Tuning().p0_tasks) {
+            want_detail = want_detail || g_stats_on;  // the step counts for the FLOPs
+            {
+                KTimer k(RL2_K_LIKELIHOOD);
+                launch_lik_task(g_stream, tg[0], most_chunks);
+            }
+            {
+                KTimer k(RL2_K_RMARG);
+                LikLaunch ra = a;
+                ra.tasks = nullptr;  // every task has ended
+                launch_rmarg(g_stream, ra);
+            }
+            copy_out();
+            if (!hip_ok(hipGetLastError(), "likelihood launch") || !q_ok) return false;
+            if (!hip_ok(hipStreamSynchronize(g_stream), "likelihood sync")) return false;
+            if (g_stats_on) count_flops();
+            give(Le, err, Lr, nit);
+            return true;
         }
         if (fused) {
             TileTask *st[2] = {b.d_tasks, b.d_tasks + (size_t)b.cap * kMaxR};
@@ -1019,10 +1059,7 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
             }
             b.tile_passes = std::min(12, std::max(2, (int)b.h_status[1] + 1));
             if (g_stats_on) stats_add_work(RL2_K_LIKELIHOOD, *b.h_flops, 0.);
-            memcpy(Le, b.h_Le, n * sizeof(double));
-            memcpy(err, b.h_err, n * sizeof(int));
-            if (Lr) memcpy(Lr, b.h_Lr, (size_t)n * kMaxR * sizeof(double));
-            if (nit) memcpy(nit, b.h_nit, (size_t)n * kMaxR * sizeof(int));
+            give(Le, err, Lr, nit);
             return true;
         }
         // Newton passes are queued ahead of the status check (the previous evaluation's
@@ -1069,20 +1106,9 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
         if (!hip_ok(hipGetLastError(), "likelihood launch")) return false;
         copy_out();
         if (!q_ok || !hip_ok(hipStreamSynchronize(g_stream), "likelihood sync")) return false;
-        if (g_stats_on) {
-            double fl = 0.;
-            for (int i = 0; i < n; i++) {
-                const double nn = o.slots[items[i].slot].n;
-                for (int r = 1; r < o.rg.numr; r++)
-                    fl += nn * (37. + 25. * b.h_nit[(size_t)i * kMaxR + r]);
-            }
-            stats_add_work(RL2_K_LIKELIHOOD, fl, 0.);
-        }
+        if (g_stats_on) count_flops();
     }
-    memcpy(Le, b.h_Le, n * sizeof(double));
-    memcpy(err, b.h_err, n * sizeof(int));
-    if (Lr) memcpy(Lr, b.h_Lr, (size_t)n * kMaxR * sizeof(double));
-    if (nit) memcpy(nit, b.h_nit, (size_t)n * kMaxR * sizeof(int));
+    give(Le, err, Lr, nit);
     return true;
 }
 
