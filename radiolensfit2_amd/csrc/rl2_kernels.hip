@@ -1116,6 +1116,86 @@ __device__ inline double read_lane(double v, int l)
     return __hiloint2double(hi, lo);
 }
 
+// Swaps of half rows of two registers: swap32 leaves {a's lanes 0-31, b's lanes 0-31} in a
+// and {a's 32-63, b's 32-63} in b; swap16 the same for each pair of rows of 16 lanes.
+__device__ inline void swap32(double &a, double &b)
+{
+    const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false,
+                                                    false);
+    const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false,
+                                                    false);
+    a = __hiloint2double((int)h[0], (int)l[0]);
+    b = __hiloint2double((int)h[1], (int)l[1]);
+}
+__device__ inline void swap16(double &a, double &b)
+{
+    const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false,
+                                                    false);
+    const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false,
+                                                    false);
+    a = __hiloint2double((int)h[0], (int)l[0]);
+    b = __hiloint2double((int)h[1], (int)l[1]);
+}
+// A lane permutation within rows that every lane takes part in.
+template <int CTRL>
+__device__ inline double dpp_perm_f64(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    const int rlo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, true);
+    const int rhi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, true);
+    return __hiloint2double(rhi, rlo);
+}
+
+// Each lane's value of the lane whose number differs in bit 2 (the other half of its eight):
+// shifts by 4 into the banks of four lanes that have a source in their half.
+__device__ inline double dpp_xor4_f64(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    int rlo = __builtin_amdgcn_update_dpp(lo, lo, 0x104, 0xf, 0x5, false);  // row_shl:4
+    int rhi = __builtin_amdgcn_update_dpp(hi, hi, 0x104, 0xf, 0x5, false);
+    rlo = __builtin_amdgcn_update_dpp(rlo, lo, 0x114, 0xf, 0xa, false);  // row_shr:4
+    rhi = __builtin_amdgcn_update_dpp(rhi, hi, 0x114, 0xf, 0xa, false);
+    return __hiloint2double(rhi, rlo);
+}
+
+// The sum of v over the eight lanes with the same lane % 8, in each of them.
+__device__ inline double wave_sum_by8(double v)
+{
+    v += dpp_perm_f64<0x128>(v);  // row_ror:8
+    double w = v;
+    swap16(v, w);
+    v += w;
+    w = v;
+    swap32(v, w);
+    return v + w;
+}
+
+// The wave's sums of eight values at once: the total of v[lane % 8] in every lane.  The lanes
+// are paired by bit 0 of their number, then bit 1, and so on, which is the order in which
+// wave_sum_last adds them (the same bits), but each of the first three steps also halves the
+// number of values that a lane holds: 10 additions with their moves instead of 48.  The seven
+// sums of a work-group by wave_sum_last took 900 cycles of a Newton pass of 5,700, and those
+// of the task's chunks as much again; with this the loop over 24 galaxies of a 64-dish array
+// went from 26.3 to 24.7 ms, batches of 16 (48 galaxies) from 15.1 to 10.5 ms, 63 points on 496
+// cells from 70.8 to 57.1 us, and 4 points on 72,000 cells from 100.5 to 97.0 us.
+__device__ inline double wave_sum8(const double (&v)[8])
+{
+    const int lane = threadIdx.x & 63;
+    double w[4], x[2];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const double keep = lane & 1 ? v[2 * k + 1] : v[2 * k];
+        w[k] = keep + dpp_perm_f64<0xb1>(lane & 1 ? v[2 * k] : v[2 * k + 1]);  // quad_perm 1032
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const double keep = lane & 2 ? w[2 * k + 1] : w[2 * k];
+        x[k] = keep + dpp_perm_f64<0x4e>(lane & 2 ? w[2 * k] : w[2 * k + 1]);  // quad_perm 2301
+    }
+    const double keep = lane & 4 ? x[1] : x[0];
+    return wave_sum_by8(keep + dpp_xor4_f64(lane & 4 ? x[0] : x[1]));
+}
+
 // The wave's maximum (MAX) or minimum in every lane, by the lane shifts of wave_sum_last; a
 // lane whose source lies outside its row, or in a row masked off, keeps its own value, which
 // leaves the extreme unchanged.  fmax and fmin are exact (and skip NaN), so the result does
@@ -1141,65 +1221,96 @@ __device__ inline double wave_extreme(double v)
     return read_lane(v, 63);
 }
 
-// The wave's inclusive prefix products, by the lane shifts of wave_sum_last; a lane without a
-// source keeps its own value (times 1).
-template <int CTRL, int ROW_MASK>
-__device__ inline double dpp_one_f64(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    const int rlo = __builtin_amdgcn_update_dpp(0, lo, CTRL, ROW_MASK, 0xf, false);
-    const int rhi = __builtin_amdgcn_update_dpp(0x3ff00000, hi, CTRL, ROW_MASK, 0xf, false);
-    return __hiloint2double(rhi, rlo);
-}
-__device__ inline double wave_scan_mul(double v)
-{
-    v *= dpp_one_f64<0x111, 0xf>(v);  // row_shr:1
-    v *= dpp_one_f64<0x112, 0xf>(v);  // row_shr:2
-    v *= dpp_one_f64<0x114, 0xf>(v);  // row_shr:4
-    v *= dpp_one_f64<0x118, 0xf>(v);  // row_shr:8
-    v *= dpp_one_f64<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-    v *= dpp_one_f64<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
-// expint_ei (rl2_math.h) by a wave, for an argument that is the same in all its lanes: lane k
-// takes the series' term k + 1.  The terms are prefix products of x / k (power series) or
-// k / x (asymptotic series, cut at its smallest term and at eps / 4), each of at most six
-// roundings where the recurrence takes 2 k, and 64 of them cost two divisions and twelve lane
-// shifts instead of a chain of 128 divisions.
-__device__ inline double expint_ei_wave(double x)
+// expint_ei (rl2_math.h) of two arguments by one wave, the same bits: the divisions of up to 64
+// terms are made by the lanes at once, and only the products and the sums that the series
+// carry from term to term run one after the other, on two lanes (one argument each) through
+// LDS.  One lane's series took two divisions a term, a hundred terms at the longest: with the
+// series on one lane the loop over 24 galaxies of a 64-dish array took 45.0 ms, with this
+// 38.5 (prefix products over the lanes took no longer, but round differently, and where few
+// points are sampled a last bit decides whether a variance is a number).
+// x0, x1 > 0 and the same in every lane; one wave of a work-group at a time (buf).
+__device__ inline void expint_ei_wave(double x0, double x1, double *y0, double *y1)
 {
     const double euler = 0.57721566490153286060651209008240243;
-    constexpr double kQuarterEps = 2.220446049250313e-16 * 0.25;
+    constexpr int U = 8;
+    __shared__ double buf[2][64];
     const int lane = threadIdx.x & 63;
-    if (x <= 40.) {
-        double sum = 0., carry = 1.;
-        for (int b = 0; b < 16; b++) {
-            const double k = (double)(64 * b + lane + 1);
-            const double p = carry * wave_scan_mul(x / k);
-            const double t = p / k;
-            sum += wave_sum(t);
-            if (read_lane(t, 63) < kQuarterEps * sum) break;
-            carry = read_lane(p, 63);
-        }
-        return euler + log(x) + sum;
+    const bool as0 = !(x0 <= 40.), as1 = !(x1 <= 40.);  // asymptotic series
+    const double *mine = buf[lane & 1];
+    double *put = buf[lane & 1];
+    // the recurrences over buf[0] and buf[1] in place, by lanes 0 and 1: c = op(c, buf[i])
+    auto chain = [&](int steps, double c, auto op) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (lane < 2)
+            for (int i = 0; i < steps; i += U) {
+                double v[U];
+#pragma unroll
+                for (int j = 0; j < U; j++) v[j] = mine[i + j];
+#pragma unroll
+                for (int j = 0; j < U; j++) {
+                    c = op(c, v[j]);
+                    put[i + j] = c;
+                }
+            }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        return c;
+    };
+    double term = 1., sum = (lane & 1 ? as1 : as0) ? 1. : 0.;  // lanes 0 and 1: carried
+    double s0 = 0., s1 = 0.;
+    bool done0 = false, done1 = false;
+    for (int base = 0; base < 1024 && !(done0 && done1); base += 64) {
+        const int steps = min(64, ((int)(2.2 * fmin(fmax(x0, x1), 40.)) + 24 + U - 1) / U * U);
+        const double k = (double)(base + lane + 1);
+        buf[0][lane] = as0 ? k / x0 : x0 / k;
+        buf[1][lane] = as1 ? k / x1 : x1 / k;
+        const double t_in = term;
+        term = chain(steps, term, [](double c, double v) { return c * v; });
+        const double p0 = buf[0][lane], p1 = buf[1][lane];
+        const double q0 = lane ? buf[0][lane - 1] : read_lane(t_in, 0);
+        const double q1 = lane ? buf[1][lane - 1] : read_lane(t_in, 1);
+        const double t0 = as0 ? p0 : p0 / k, t1 = as1 ? p1 : p1 / k;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        buf[0][lane] = t0;
+        buf[1][lane] = t1;
+        const double s_in = sum;
+        sum = chain(steps, sum, [](double c, double v) { return c + v; });
+        // the first term at which the series ends: with it (below eps / 4 of the sum), or
+        // before it (an asymptotic term no smaller than the one before)
+        auto end = [&](const double *S, double t, double q, bool as, double in, double *s) {
+            const double sl = S[lane];
+            const bool before = as && t >= q;
+            const uint64_t m =
+                __ballot(lane < steps && (before || t < 2.220446049250313e-16 * 0.25 * sl));
+            const int f = m ? __ffsll((unsigned long long)m) - 1 : steps - 1;
+            const bool b = m && ((__ballot(before) >> f) & 1);
+            *s = b ? (f ? read_lane(sl, f - 1) : in) : read_lane(sl, f);
+            return m != 0;
+        };
+        double s;
+        const bool e0 = end(buf[0], t0, q0, as0, read_lane(s_in, 0), &s);
+        if (!done0) s0 = s;
+        done0 = done0 || e0;
+        const bool e1 = end(buf[1], t1, q1, as1, read_lane(s_in, 1), &s);
+        if (!done1) s1 = s;
+        done1 = done1 || e1;
+        if (steps < 64 && !(done0 && done1)) base -= 64 - steps;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    const double k = (double)(lane + 1);
-    const double t = wave_scan_mul(k / x);
-    const double sum = 1. + wave_sum(k < x && t >= kQuarterEps ? t : 0.);
-    return exp(x) / x * sum;
+    *y0 = as0 ? exp(x0) / x0 * s0 : euler + log(x0) + s0;
+    *y1 = as1 ? exp(x1) / x1 * s1 : euler + log(x1) + s1;
 }
 
-// marg_position (rl2_math.h) by a wave, for an argument that is the same in all its lanes.
-// The two exponential integrals were the longest serial chain of a task that ends with
-// B <= 100 (a hundred dependent divisions each, by one lane).
+// marg_position (rl2_math.h) by a wave, for an argument that is the same in all its lanes,
+// with the same bits.  The two exponential integrals of a task that ends with B <= 100 were its
+// longest serial chain, by one lane, on the critical path of the Newton pass.
 __device__ inline double marg_position_wave(double x)
 {
     const double Delta = 0.5 * 5.991;
     if (x <= Delta) return kBad;
     if (x > 100.) return x - log(Delta) - exp(-Delta);
     if ((x - Delta) < 0.0001) x = Delta + 0.0001;
-    const double yc = expint_ei_wave(x), ys = expint_ei_wave(x - Delta);
+    double yc, ys;
+    expint_ei_wave(x, x - Delta, &yc, &ys);
     return log((yc - ys) / log(x / (x - Delta)));
 }
 
@@ -2834,47 +2945,53 @@ __device__ int newton_update(TileTask &T, const double (&v)[7], double *ho_out,
     return 1;
 }
 
-// finish_lr of a step that a whole wave took, when lane 63, which holds the task's totals,
-// ended the task: its values go to every lane for the wave-parallel position marginalisation.
-__device__ inline void finish_lane63(const LikLaunch &a, int item, int r, int done, double ho,
-                                     double det, int iter)
-{
-    if (__builtin_amdgcn_readlane(done, 63))
-        finish_lr(a, item, r, read_lane(ho, 63), read_lane(det, 63),
-                  __builtin_amdgcn_readlane(iter, 63));
-}
-
 // newton_update on the task's state in memory, writing L_r when the task finishes (the
 // step kernel of the two-kernel passes).
 // The state is read from T and written to To (the same task in another buffer when the
-// passes keep two generations of state; T itself otherwise).  Called by a whole wave whose
-// lane 63 holds the sums; that lane writes the state, and its return value and offset count.
+// passes keep two generations of state; T itself otherwise).  Called by a whole wave with the
+// same sums in every lane; lane 0 writes the state.
 template <int PASS>
 __device__ int tile_step(const LikLaunch &a, const TileTask *T, TileTask *To, int item, int r,
                          const double (&v)[7], double *xo, double *yo)
 {
     TileTask S = *T;
-    double ho = 0., det = 0.;
+    double ho, det;
     const int done = newton_update<PASS>(S, v, &ho, &det);
-    if ((threadIdx.x & 63) == 63) *To = S;
-    finish_lane63(a, item, r, done, ho, det, S.iter);
+    if ((threadIdx.x & 63) == 0) *To = S;
+    if (done) finish_lr(a, item, r, ho, det, S.iter);
     *xo = S.xo;
     *yo = S.yo;
     return done;
 }
 
-// A task's chunk sums of one pass added in chunk order by one wave: lanes over chunks, then
-// across lanes into lane 63.  P0 is the task's first chunk; chunk c follows at c * nr * 8.
+// A task's chunk sums of one pass added by one wave in a fixed order, with the totals in every
+// lane: the chunks are paired by bit 0 of their number (mod 64), then bit 1, and so on.  Lane l
+// reads value l % 8 of chunks 8 i + l / 8 (and those 64, 128, ... further, added first) for
+// each block i of eight chunks; a block adds up over its lanes, then the blocks by pairs.
+// read(i, c): the lane's sum over the chunks c, c + 64, ... below nch of block i.
+template <class Read>
+__device__ inline void task_totals(unsigned nch, const Read &read, double (&v)[7])
+{
+    const int lane = threadIdx.x & 63;
+    double t[8];
+#pragma unroll
+    for (unsigned i = 0; i < 8; i++)
+        t[i] = 8 * i < nch ? wave_sum_by8(read(i, 8 * i + (lane >> 3))) : 0.;
+    const double s = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+#pragma unroll
+    for (int j = 0; j < 7; j++) v[j] = read_lane(s, j);
+}
+// P0 is the task's first chunk; chunk c follows at c * nr * 8.
 __device__ inline void task_sums(const double *P0, unsigned nch, int nr, int lane,
                                  double (&v)[7])
 {
-#pragma unroll
-    for (int j = 0; j < 7; j++) v[j] = 0.;
-    for (unsigned c = lane; c < nch; c += 64)
-#pragma unroll
-        for (int j = 0; j < 7; j++) v[j] += P0[(size_t)c * nr * 8 + j];
-#pragma unroll
-    for (int j = 0; j < 7; j++) v[j] = wave_sum_last(v[j]);  // totals in lane 63
+    task_totals(nch,
+                [&](unsigned, unsigned c) {
+                    double t = 0.;
+                    for (; c < nch; c += 64) t += P0[(size_t)c * nr * 8 + (lane & 7)];
+                    return t;
+                },
+                v);
 }
 
 // Newton phase tables e^{2 pi i o ctr[k]} (o = xo for the columns, yo for the rows) by runs
@@ -2942,23 +3059,20 @@ __device__ inline double2 tab_y(const TabRot<NRUN> &R, unsigned k)
     return tab_entry(R.ey[k / kTabRun], R.wy[k % kTabRun]);
 }
 
-// The chunk sums of a tile work-group into P[0..N-1]: each wave's total from lane 63, then
-// thread j adds the waves' value j in wave order.
-template <int N>
-__device__ inline void tile_reduce(double (&v)[N], double *lds, double *P)
+// The chunk sums of a tile work-group into P[0..7]: each wave's totals, then thread j adds the
+// waves' value j in wave order.
+__device__ inline void tile_reduce(double (&v)[7], double *lds, double *P)
 {
     constexpr int NW = kTileBS / 64;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-    for (int j = 0; j < N; j++) v[j] = wave_sum_last(v[j]);
-    if (lane == 63)
-#pragma unroll
-        for (int j = 0; j < N; j++) lds[wave * N + j] = v[j];
+    double w[8] = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], 0.};
+    const double s = wave_sum8(w);
+    if (lane < 8) lds[wave * 8 + lane] = s;
     __syncthreads();
-    if (threadIdx.x < N) {
+    if (threadIdx.x < 8) {
         double t = 0.;
 #pragma unroll
-        for (int q = 0; q < NW; q++) t += lds[q * N + threadIdx.x];
+        for (int q = 0; q < NW; q++) t += lds[q * 8 + threadIdx.x];
         P[threadIdx.x] = t;
     }
     __syncthreads();  // lds is reused by the block's next logical work-group
@@ -3102,13 +3216,11 @@ __device__ inline void tile_chunk(const TileLaunch &t, unsigned wg, double *red)
             tile_sums32<PASS>(F, it, a.rg.ro[r], PASS == 1 ? T->xo : 0.,
                               PASS == 1 ? T->yo : 0., beg, end, s);
     }
-    tile_reduce<7>(s, red, t.partials + (size_t)wg * 8);
+    tile_reduce(s, red, t.partials + (size_t)wg * 8);
 }
 
-// One work-group per (item, r) task.  Wave 0 adds the task's chunk sums in a fixed order
-// (lanes over chunks, then across lanes into lane 63), and lane 63 takes the Newton step or
-// ends the task; when
-// the task goes on over a grid facet in FP64, the whole group (16 waves, so each lane
+// One work-group per (item, r) task.  Wave 0 adds the task's chunk sums in a fixed order and
+// takes the Newton step or ends the task; when the task goes on over a grid facet in FP64, the whole group (16 waves, so each lane
 // writes at most 3 entries of the 2 * facet) then writes its phase tables for the next pass.
 constexpr int kStepBS = 1024;
 template <int PASS>
@@ -3132,7 +3244,7 @@ __global__ __launch_bounds__(kStepBS) void lik_step_kernel(TileLaunch t)
     if (threadIdx.x < 64) {
         const int lane = threadIdx.x;
         int go = 0;
-        if (PASS == 0 || T->active) {  // read by the whole wave before lane 63 updates it
+        if (PASS == 0 || T->active) {  // read by the whole wave before lane 0 updates it
             unsigned first, nch;
             tile_range(t, a.items, item, &first, &nch);
             double v[7];
@@ -3140,14 +3252,14 @@ __global__ __launch_bounds__(kStepBS) void lik_step_kernel(TileLaunch t)
                       v);
             double xo, yo;
             go = !tile_step<PASS>(a, T, To, item, r, v, &xo, &yo);
-            if (lane == 63) {
+            if (lane == 0) {
                 s_off[0] = xo;
                 s_off[1] = yo;
             }
-        } else if (lane == 63 && To != T) {
+        } else if (lane == 0 && To != T) {
             *To = *T;  // a finished task keeps its state in the other generation too
         }
-        if (lane == 63) s_go = go;
+        if (lane == 0) s_go = go;
     }
     __syncthreads();
     if (!s_go || !t.tab) return;
@@ -3197,10 +3309,11 @@ __device__ void tile_status(const LikLaunch &a)
 // What a fused pass's work-group reads of its task before anything else, so that these
 // loads are in flight with the facet's and the cells': the task's state S (the same address
 // in every thread: scalar loads) and wave 0's share of the previous pass's chunk sums of the
-// task (lane c: chunk c, when nch <= 64; task_sums reads them itself otherwise).
+// task (task_sums' lanes, when nch <= 8 kPreChunks; task_sums reads them itself otherwise).
+constexpr unsigned kPreChunks = 4;
 struct FusedPre {
     TileTask S;
-    double p[7];
+    double p[kPreChunks];
 };
 
 __device__ __attribute__((always_inline)) inline FusedPre fused_pre(const TileLaunch &t,
@@ -3210,14 +3323,14 @@ __device__ __attribute__((always_inline)) inline FusedPre fused_pre(const TileLa
 {
     FusedPre f;
     f.S = t.tasks[(size_t)item * kMaxR + r];
-#pragma unroll
-    for (int j = 0; j < 7; j++) f.p[j] = 0.;
     const unsigned lane = threadIdx.x;
-    if (t.mode != 2 && nch <= 64 && lane < nch) {
-        const double *P = t.part_in + (size_t)(first + (unsigned)(r - t.r_lo)) * 8 +
-                          (size_t)lane * t.nr_g * 8;
+    const bool read = t.mode != 2 && nch <= 8 * kPreChunks && lane < 64;
+    const double *P = t.part_in + (size_t)(first + (unsigned)(r - t.r_lo)) * 8 + (lane & 7);
 #pragma unroll
-        for (int j = 0; j < 7; j++) f.p[j] = P[j];
+    for (unsigned k = 0; k < kPreChunks; k++) {
+        const unsigned c = (lane >> 3) + 8 * k;
+        f.p[k] = 0.;
+        if (read && 8 * k < nch && c < nch) f.p[k] = P[(size_t)c * t.nr_g * 8];
     }
     return f;
 }
@@ -3244,34 +3357,32 @@ __device__ __attribute__((always_inline)) inline void fused_step(const TileLaunc
         yo = pre.S.yo;
     } else {
         double v[7];
-        if (nch <= 64) {  // task_sums' arithmetic on the chunk sums read at the start
-#pragma unroll
-            for (int j = 0; j < 7; j++) {
-                double pj = pre.p[j];
-                asm volatile("" : "+v"(pj));  // consumed here, not where the load was issued
-                v[j] = 0.;
-                v[j] += pj;
-            }
-#pragma unroll
-            for (int j = 0; j < 7; j++) v[j] = wave_sum_last(v[j]);
+        if (nch <= 8 * kPreChunks) {  // task_sums' arithmetic on the chunk sums read at the start
+            task_totals(nch,
+                        [&](unsigned i, unsigned) {
+                            double p = i < kPreChunks ? pre.p[i < kPreChunks ? i : 0] : 0.;
+                            asm volatile("" : "+v"(p));  // consumed here, not at the load's issue
+                            return p;
+                        },
+                        v);
         } else {
             task_sums(t.part_in + (size_t)(first + (unsigned)(r - t.r_lo)) * 8, nch, t.nr_g,
                       lane, v);
         }
-        // the totals, and so the step, are lane 63's: the other lanes take it on partial sums
+        // every lane takes the step from the same totals: the end of a task is the wave's
         TileTask S = t.mode == 0 ? TileTask{} : pre.S;
-        double ho = 0., det = 0.;
+        double ho, det;
         const int done = t.mode == 0 ? newton_update<0>(S, v, &ho, &det)
                                      : newton_update<1>(S, v, &ho, &det);
         if (chunk == 0) {
-            if (lane == 63) t.tasks_out[ti] = S;
-            finish_lane63(a, item, r, done, ho, det, S.iter);
+            if (lane == 0) t.tasks_out[ti] = S;
+            if (done) finish_lr(a, item, r, ho, det, S.iter);
         }
         go = !done;
         xo = S.xo;
         yo = S.yo;
     }
-    if (lane == 63) {
+    if (lane == 0) {
         *go_out = go;
         off[0] = xo;
         off[1] = yo;
@@ -3401,7 +3512,7 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_fused_kernel(Tile
     double s[7];
     if (tile_sums64_rec(fn, loff, dc, it, a.rg.ro[r], make, reinterpret_cast<const char *>(rec),
                         beg, end, s))
-        tile_reduce<7>(s, red, t.partials + (size_t)wg * 8);
+        tile_reduce(s, red, t.partials + (size_t)wg * 8);
 }
 
 // ------------------------------------------------------------------ one launch per evaluation
@@ -3410,23 +3521,19 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_fused_kernel(Tile
 // completed, and only then counts the chunk as done on the task's counter.  A reader that
 // sees the count loads the sums at agent scope too.  Every sum lives at its own address for
 // the whole launch (one slice per pass), so no reader can hold an older copy of it.
-template <int N>
-__device__ inline void tile_reduce_publish(double (&v)[N], double *lds, double *P,
-                                           unsigned *cnt)
+__device__ inline void tile_reduce_publish(double (&v)[7], double *lds, double *P, unsigned *cnt)
 {
     constexpr int NW = kTileBS / 64;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-    for (int j = 0; j < N; j++) v[j] = wave_sum_last(v[j]);
-    if (lane == 63)
-#pragma unroll
-        for (int j = 0; j < N; j++) lds[wave * N + j] = v[j];
+    double w[8] = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], 0.};
+    const double s = wave_sum8(w);
+    if (lane < 8) lds[wave * 8 + lane] = s;
     __syncthreads();
     if (threadIdx.x < 64) {
-        if (threadIdx.x < N) {
+        if (threadIdx.x < 8) {
             double t = 0.;
 #pragma unroll
-            for (int q = 0; q < NW; q++) t += lds[q * N + threadIdx.x];
+            for (int q = 0; q < NW; q++) t += lds[q * 8 + threadIdx.x];
             __hip_atomic_store(P + threadIdx.x, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -3441,15 +3548,15 @@ __device__ inline void tile_reduce_publish(double (&v)[N], double *lds, double *
 __device__ inline void task_sums_published(const double *P0, unsigned nch, int nr, int lane,
                                            double (&v)[7])
 {
-#pragma unroll
-    for (int j = 0; j < 7; j++) v[j] = 0.;
-    for (unsigned c = lane; c < nch; c += 64)
-#pragma unroll
-        for (int j = 0; j < 7; j++)
-            v[j] += __hip_atomic_load(P0 + (size_t)c * nr * 8 + j, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-    for (int j = 0; j < 7; j++) v[j] = wave_sum_last(v[j]);  // totals in lane 63
+    task_totals(nch,
+                [&](unsigned, unsigned c) {
+                    double t = 0.;
+                    for (; c < nch; c += 64)
+                        t += __hip_atomic_load(P0 + (size_t)c * nr * 8 + (lane & 7),
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    return t;
+                },
+                v);
 }
 
 // One block's share of an evaluation: a task, and the run of its chunks the block sums.
@@ -3573,17 +3680,17 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_persist_kernel(Pe
                                                   (unsigned)(K.r - 1)) * 8,
                                         K.nch, nr, lane, v);
                     TileTask S = pass == 1 ? TileTask{} : K.S;
-                    double ho = 0., det = 0.;
+                    double ho, det;
                     const int done = pass == 1 ? newton_update<0>(S, v, &ho, &det)
                                                : newton_update<1>(S, v, &ho, &det);
-                    if (lane == 63) {
+                    if (lane == 0) {
                         K.S = S;
                         K.active = !done;
                         if (done && K.c0 == 0) p.t.tasks[ti] = S;
                         s_off[0] = S.xo;
                         s_off[1] = S.yo;
                     }
-                    if (K.c0 == 0) finish_lane63(a, K.item, K.r, done, ho, det, S.iter);
+                    if (done && K.c0 == 0) finish_lr(a, K.item, K.r, ho, det, S.iter);
                 }
                 __syncthreads();
                 if (!K.active) continue;
@@ -3619,7 +3726,7 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_persist_kernel(Pe
                 auto none = []() { return true; };  // the records are already staged
                 tile_sums64_rec(F.n, F.loff, F.dc, it, ro, none,
                                 reinterpret_cast<const char *>(rec), beg, end, s);
-                tile_reduce_publish<7>(
+                tile_reduce_publish(
                     s, red, p.part + ((size_t)pass * t.nwg + K.first + c * nr + (K.r - 1)) * 8,
                     p.cnt + ti);
             }
@@ -3646,10 +3753,10 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_persist_kernel(Pe
 // 96 here; from 8,192 cells on (twice the cells in registers, which spill) 71, 77 and 128
 // against 75, 76 and 139, so kTaskChunks is 4.
 template <int KIND, int G, int NC>
-__global__ __launch_bounds__(kTileBS *G) void lik_task_kernel(TileLaunch t)
+__global__ __launch_bounds__(kTileBS *G, NC == 1 ? 3 : 2) void lik_task_kernel(TileLaunch t)
 {
     constexpr int BS = kTileBS * G, Q = kTileMinCells / kTileBS, W = kTileBS / 64;
-    constexpr int NJ = 7;
+    constexpr int NJ = 8;
     __shared__ double red[G * NC][W][NJ];
     __shared__ TabRot<kRecFacet / kTabRun> R;
     extern __shared__ double2 tab_lds[];  // t.tab_lds_facet records
@@ -3701,15 +3808,10 @@ __global__ __launch_bounds__(kTileBS *G) void lik_task_kernel(TileLaunch t)
     const double sw = sf * (4 * kPi * kPi);
     const double a1 = 1. + e1, a2 = 1. - e1;
     constexpr double kTwoPi2 = kTwoPi * kTwoPi;
-    // a chunk's sums of this wave, from lane 63
-    auto put = [&](int k, double (&s)[NJ], int nj) {
-#pragma unroll
-        for (int j = 0; j < NJ; j++)
-            if (j < nj) s[j] = wave_sum_last(s[j]);
-        if (lane == 63)
-#pragma unroll
-            for (int j = 0; j < NJ; j++)
-                if (j < nj) red[g + k * G][wave][j] = s[j];
+    // a chunk's sums of this wave
+    auto put = [&](int k, double (&s)[NJ]) {
+        const double x = wave_sum8(s);
+        if (lane < 8) red[g + k * G][wave][lane] = x;
     };
 #pragma unroll
     for (int k = 0; k < NC; k++) {  // pass 0: tile_sums64_p0_db's terms
@@ -3741,34 +3843,30 @@ __global__ __launch_bounds__(kTileBS *G) void lik_task_kernel(TileLaunch t)
         s[4] *= kTwoPi2;
         s[5] *= kTwoPi2;
         s[6] *= kTwoPi2;
-        put(k, s, 7);
+        put(k, s);
     }
     TileTask S = {};
+    double ho, det;
     for (int pass = 0;; pass++) {
         __syncthreads();
         // every wave adds the task's chunk sums (tile_reduce's order over the waves, then
-        // task_sums' over the chunks) and takes the step from lane 63's totals
-        double v[NJ];
+        // task_sums' over the chunks) and takes the step
+        static_assert(G * NC <= 8, "one block of chunks");
+        double v[7];
+        task_totals(min(nch, (unsigned)(G * NC)),
+                    [&](unsigned, unsigned c) {
+                        double p = 0.;
+                        if (c < nch && c < G * NC) {
 #pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            double p = 0.;
-            if (lane < (int)nch) {
-#pragma unroll
-                for (int w = 0; w < W; w++) p += red[lane < G * NC ? lane : 0][w][j];
-            }
-            v[j] = 0.;
-            v[j] += p;
-            v[j] = wave_sum_last(v[j]);
-        }
-        double ho = 0., det = 0.;
+                            for (int w = 0; w < W; w++) p += red[c][w][lane & 7];
+                        }
+                        return p;
+                    },
+                    v);
         const int done = pass == 0 ? newton_update<0>(S, v, &ho, &det)
                                    : newton_update<1>(S, v, &ho, &det);
-        if (__builtin_amdgcn_readlane(done, 63)) {  // the same in every wave
-            if (threadIdx.x < 64) finish_lane63(a, item, r, done, ho, det, S.iter);
-            return;
-        }
-        const double xo = read_lane(S.xo, 63), yo = read_lane(S.yo, 63);
-        tab_rot_stage(R, RecCtr{rec}, gf, xo, yo, 0u, (gf + kTabRun - 1) / kTabRun - 1, false);
+        if (done) break;  // the same in every wave
+        tab_rot_stage(R, RecCtr{rec}, gf, S.xo, S.yo, 0u, (gf + kTabRun - 1) / kTabRun - 1, false);
         __syncthreads();
         for (unsigned q = threadIdx.x; q < 2 * gf; q += BS) {
             const unsigned k = q < gf ? q : q - gf;
@@ -3806,9 +3904,10 @@ __global__ __launch_bounds__(kTileBS *G) void lik_task_kernel(TileLaunch t)
             s[3] *= kTwoPi2;
             s[4] *= kTwoPi2;
             s[5] *= kTwoPi2;
-            put(k, s, 6);
+            put(k, s);
         }
     }
+    if (threadIdx.x < 64) finish_lr(a, item, r, ho, det, S.iter);
 }
 
 template <int KIND>
@@ -4028,7 +4127,7 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_fused_wide_kernel
                                        end, s)
                : tile_sums64_col<false>(F, it, a.rg.ro[r], make, col, sY, R, row_lo, span, beg,
                                         end, s);
-    if (ran) tile_reduce<7>(s, red, t.partials + (size_t)wg * 8);
+    if (ran) tile_reduce(s, red, t.partials + (size_t)wg * 8);
 }
 
 void launch_tile_fused(hipStream_t s, const TileLaunch &t)
@@ -4079,7 +4178,7 @@ __device__ inline void p0_group_chunk(const TileLaunch &t, const LikItem *items,
     tile_sums64_p0_db<NT>(F, it, ro, sC, stage, beg, end, s);
     const size_t w0 = (size_t)cg * (unsigned)t.nr_g + (unsigned)(ra - t.r_lo);
 #pragma unroll
-    for (int q = 0; q < NT; q++) tile_reduce<7>(s[q], red, t.partials + (w0 + q) * 8);
+    for (int q = 0; q < NT; q++) tile_reduce(s[q], red, t.partials + (w0 + q) * 8);
 }
 
 template <int KIND, int TPW>
@@ -4193,18 +4292,17 @@ void launch_marginalise_r(hipStream_t s, int num, const double *x, const double 
 
 // marg_position (likelihood.c:376-421) on n given arguments, one per wave: the device
 // function finish_lr applies to B = ho^2 / 2.
-__global__ __launch_bounds__(256) void marg_position_kernel(int n, const double *x, double *out)
+__global__ __launch_bounds__(64) void marg_position_kernel(int n, const double *x, double *out)
 {
-    const int i = blockIdx.x * (256 / 64) + (threadIdx.x >> 6);
-    if (i >= n) return;  // a whole wave
+    const int i = blockIdx.x;
     const double y = marg_position_wave(x[i]);
-    if ((threadIdx.x & 63) == 0) out[i] = y;
+    if (threadIdx.x == 0) out[i] = y;
 }
 
 void launch_marg_position(hipStream_t s, int n, const double *x, double *out)
 {
     if (n <= 0) return;
-    marg_position_kernel<<<(n + 3) / 4, 256, 0, s>>>(n, x, out);
+    marg_position_kernel<<<n, 64, 0, s>>>(n, x, out);
 }
 
 // ------------------------------------------------------------------ subtraction (K2)
