@@ -265,6 +265,9 @@ struct LikLaunch {
     double *det = nullptr;     // optional nitems * kMaxR: Hessian determinant at the peak
     const int *host_prec = nullptr;  // host copy of items[].prec (selects the kernels)
     const TileTask *tasks = nullptr; // tiled engine: per-(item, r) state (fragile flags)
+    // optional: L_r and the step counts in pinned host memory too (nitems * kMaxR each)
+    double *Lr_host = nullptr;
+    int *nit_host = nullptr;
     // tiled engine: the r-marginalisation launch also writes the evaluation's status
     // (tasks still iterating, largest step count) and FLOP-equivalents when set
     unsigned *status = nullptr;
@@ -325,6 +328,9 @@ struct TileLaunch {
     // previous pass's sums read from `part_in` while this pass's go to `partials`.
     TileTask *tasks_out = nullptr;
     const double *part_in = nullptr;
+    // lik_task_kernel with the items in the arguments: tasks ended per item, zero before the
+    // launch, and the launch leaves them zero again
+    unsigned *arrived = nullptr;
     int mode = 0;              // fused passes: 0 first step (from the pass-0 sums), 1 Newton
                                // step, 2 resume from the state in `tasks`
     unsigned item_chunks = 0;  // chunks of every item when all items have the same count
@@ -332,7 +338,8 @@ struct TileLaunch {
 };
 void launch_tile_pass(hipStream_t s, const TileLaunch &t, int pass);
 // Every pass of every task in one launch: items of at most kTaskChunks chunks of
-// kTileMinCells cells (chunks: the largest), on grid facets with records.
+// kTileMinCells cells (chunks: the largest), on grid facets with records; with the items in
+// the kernel arguments (grid 2) the r-marginalisation too.
 constexpr unsigned kTaskChunks = 4;
 void launch_lik_task(hipStream_t s, const TileLaunch &t, unsigned chunks);
 // One Newton pass with the previous pass's step folded in (grid items, row tables in LDS).

@@ -1334,6 +1334,10 @@ __device__ inline void finish_lr(const LikLaunch &a, int item, int r, double ho,
     if ((threadIdx.x & 63) != 0) return;
     a.Lr[(size_t)item * kMaxR + r] = L;
     a.nit[(size_t)item * kMaxR + r] = iter;
+    if (a.Lr_host) {  // pinned memory: the caller reads them after its one synchronisation
+        a.Lr_host[(size_t)item * kMaxR + r] = L;
+        a.nit_host[(size_t)item * kMaxR + r] = iter;
+    }
     if (a.ho) a.ho[(size_t)item * kMaxR + r] = ho;
     if (a.det) a.det[(size_t)item * kMaxR + r] = det_sigma;
 }
@@ -2222,14 +2226,14 @@ __device__ int qag41_wave(const SplineLds &sp, const Gk41Node &g, double a, doub
 // points above kBad go, in r order, to knots 0..num-1 in LDS; ymax, xmin and xmax are wave
 // reductions (xmin and xmax are the extreme abscissae: the reference's start from the
 // neighbours of the maximum does not change them); the QUADPACK lists live in LDS.
-__device__ void rmarg_item(const LikLaunch &a, int item, SplineLds &sp, double *qd, int *qi)
+__device__ void rmarg_item(const LikLaunch &a, const LikItem &it, int item, SplineLds &sp,
+                           double *qd, int *qi)
 {
     const int lane = threadIdx.x & 63;
     const int numR = a.rg.numr;
     const bool mine = lane >= 1 && lane < numR;
     // every global read of the item is issued here, the node tables first
     const Gk41Node g = gk41_node();
-    const LikItem it = a.items[item];
     const size_t base = (size_t)item * kMaxR;
     const double lv = mine ? a.Lr[base + lane] : kBad;
     bool act = false, frag = false;
@@ -2307,7 +2311,7 @@ __global__ __launch_bounds__(128) void rmarg_kernel(LikLaunch a)
     __shared__ SplineLds sp;
     __shared__ double qd[kQagDoubles];
     __shared__ int qi[kQagInts];
-    rmarg_item(a, blockIdx.x, sp, qd, qi);
+    rmarg_item(a, a.items[blockIdx.x], blockIdx.x, sp, qd, qi);
 }
 
 // ------------------------------------------------------------------ likelihood, tiled
@@ -3747,6 +3751,10 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_persist_kernel(Pe
 // the chunk sums, the step and the table entries are those of pass 0 and the fused passes, so
 // every L_r is the same bit for bit by either route.
 // G groups of 256 threads; a task has at most G * NC chunks (chunk c: group c % G).
+// KIND 2 (up to kInlItems items, in the arguments): the work-group that ends an item's last
+// task also integrates over the scalelength (rmarg_item), so an evaluation is one launch.
+// With more items its lists (40 KB of LDS) would cost the task work-groups their residency,
+// and a launch of their own is a small part of the evaluation.
 // Measured against the passes: one point on 138 cells 64.1 -> 46.5 us, the loop over 24
 // galaxies of 175 to 2111 cells 38.5 -> 26.3 ms, in batches of 16 (48 galaxies) 18.4 -> 15.1
 // ms.  On 6,582 cells 1, 4 and 24 points took 69, 71 and 102 us by the passes and 60, 60 and
@@ -3762,8 +3770,6 @@ __global__ __launch_bounds__(kTileBS *G, NC == 1 ? 3 : 2) void lik_task_kernel(T
     extern __shared__ double2 tab_lds[];  // t.tab_lds_facet records
     RecEntry *rec = reinterpret_cast<RecEntry *>(tab_lds);
     const char *recb = reinterpret_cast<const char *>(tab_lds);
-    if (KIND == 2 && blockIdx.x == 0 && threadIdx.x < t.n_inl)
-        t.items_w[threadIdx.x] = t.inl[threadIdx.x];
     const LikLaunch &a = t.lk;
     const int item = (int)(blockIdx.x / (unsigned)t.nr_g);
     const int r = (int)(blockIdx.x - (unsigned)item * (unsigned)t.nr_g) + t.r_lo;
@@ -3908,12 +3914,32 @@ __global__ __launch_bounds__(kTileBS *G, NC == 1 ? 3 : 2) void lik_task_kernel(T
         }
     }
     if (threadIdx.x < 64) finish_lr(a, item, r, ho, det, S.iter);
+    if constexpr (KIND == 2) {
+        __shared__ SplineLds sp;
+        __shared__ bool s_last;
+        if (threadIdx.x >= 128) return;
+        if (threadIdx.x == 0) {
+            // lane 0 wrote L_r: released with this count, and the other tasks' acquired
+            const unsigned k = __hip_atomic_fetch_add(t.arrived + item, 1u, __ATOMIC_ACQ_REL,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+            s_last = k + 1 == (unsigned)t.nr_g;
+            if (s_last)  // zero again for the next launch
+                __hip_atomic_store(t.arrived + item, 0u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        if (!s_last) return;
+        double *qd = reinterpret_cast<double *>(tab_lds);  // the records are done with
+        rmarg_item(a, it, item, sp, qd, reinterpret_cast<int *>(qd + kQagDoubles));
+    }
 }
 
 template <int KIND>
 static void launch_task_kind(hipStream_t s, const TileLaunch &t, unsigned chunks)
 {
-    const unsigned g = (unsigned)t.lk.nitems * (unsigned)t.nr_g, lds = t.tab_lds_facet * kRecBytes;
+    const unsigned g = (unsigned)t.lk.nitems * (unsigned)t.nr_g;
+    unsigned lds = t.tab_lds_facet * kRecBytes;
+    if (KIND == 2) lds = std::max(lds, (unsigned)(kQagDoubles * 8 + kQagInts * 4));
     if (chunks <= 1)
         lik_task_kernel<KIND, 1, 1><<<g, kTileBS, lds, s>>>(t);
     else if (chunks <= 2)

@@ -53,6 +53,9 @@ struct LikBuffers {
     double *d_ppart = nullptr;                           // one-launch evaluations: chunk
     size_t ppart_cap = 0;                                // sums per pass (work-groups)
     unsigned *d_cnt = nullptr;                           // cap * kMaxR chunk counters
+    unsigned *d_arrived = nullptr;                       // kInlItems task counters
+    double *d_Lr_host = nullptr;                         // device views of h_Lr, h_nit
+    int *d_nit_host = nullptr;
     double2 *d_tab = nullptr;                            // Newton phase tables
     size_t tab_cap = 0;                                  // entries
     int tile_passes = 6;     // Newton passes queued before the first status check

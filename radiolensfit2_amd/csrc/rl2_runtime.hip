@@ -171,7 +171,9 @@ bool LikBuffers::ensure(int n)
               dmalloc(&d_nit, (size_t)c * kMaxR) &&
               dmalloc(&d_ws, (size_t)c * kQagDoubles) && dmalloc(&d_iws, (size_t)c * kQagInts) &&
               dmalloc(&d_tasks, (size_t)c * kMaxR * 2) &&  // two generations of task state
-              dmalloc(&d_cnt, (size_t)c * kMaxR);
+              dmalloc(&d_cnt, (size_t)c * kMaxR) && dmalloc(&d_arrived, kInlItems);
+    ok = ok && hip_ok(hipMemsetAsync(d_arrived, 0, kInlItems * sizeof(unsigned), g_stream),
+                      "memset");
     ok = ok && hip_ok(hipMemsetAsync(d_tasks, 0, (size_t)c * kMaxR * 2 * sizeof(TileTask),
                                      g_stream),
                       "memset");
@@ -181,7 +183,9 @@ bool LikBuffers::ensure(int n)
          hip_ok(hipHostGetDevicePointer((void **)&d_out, h_out, 0), "hipHostGetDevicePointer") &&
          hip_ok(hipHostMalloc((void **)&h_items, c * sizeof(LikItem)), "hipHostMalloc") &&
          hip_ok(hipHostMalloc((void **)&h_Lr, (size_t)c * kMaxR * sizeof(double)), "hipHostMalloc") &&
-         hip_ok(hipHostMalloc((void **)&h_nit, (size_t)c * kMaxR * sizeof(int)), "hipHostMalloc");
+         hip_ok(hipHostMalloc((void **)&h_nit, (size_t)c * kMaxR * sizeof(int)), "hipHostMalloc") &&
+         hip_ok(hipHostGetDevicePointer((void **)&d_Lr_host, h_Lr, 0), "hipHostGetDevicePointer") &&
+         hip_ok(hipHostGetDevicePointer((void **)&d_nit_host, h_nit, 0), "hipHostGetDevicePointer");
     if (!ok) return false;
     cap = c;
     d_status = (unsigned *)d_out;
@@ -204,6 +208,9 @@ void LikBuffers::release()
     dfree(d_iws);
     dfree(d_tasks);
     dfree(d_cnt);
+    dfree(d_arrived);
+    d_Lr_host = nullptr;
+    d_nit_host = nullptr;
     if (h_out) (void)hipHostFree(h_out);
     if (h_items) (void)hipHostFree(h_items);
     if (h_Lr) (void)hipHostFree(h_Lr);
@@ -750,21 +757,16 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
     bool tiled = o.lik_block == 0;
     for (int i = 0; i < n && tiled; i++)
         if (o.h_facets[items[i].slot].mod) tiled = false;  // given model: one group per (e, r)
-    bool want_detail = Lr || nit || (g_stats_on && !tiled);
     // Every copy, fill and stream dependency queued below ANDs its status into q_ok, which
     // is checked with the launches' before the results are read.
     bool q_ok = true;
-    // one copy back per evaluation: status, FLOP count, L_e and the error flags
-    auto copy_out = [&]() {  // the results block itself is written to host memory
-        if (want_detail)
-            q_ok = hip_ok(hipMemcpyAsync(b.h_Lr, b.d_Lr, (size_t)n * kMaxR * sizeof(double),
-                                         hipMemcpyDeviceToHost, g_stream),
-                          "L_r copy") &&
-                   hip_ok(hipMemcpyAsync(b.h_nit, b.d_nit, (size_t)n * kMaxR * sizeof(int),
-                                         hipMemcpyDeviceToHost, g_stream),
-                          "step count copy") &&
-                   q_ok;
+    // The results (status, FLOP count, L_e, error flags, and on request L_r and the step
+    // counts) are written to pinned host memory by the kernels: nothing is copied back.
+    auto want_detail = [&](bool want) {
+        a.Lr_host = want ? b.d_Lr_host : nullptr;
+        a.nit_host = want ? b.d_nit_host : nullptr;
     };
+    want_detail(Lr || nit || (g_stats_on && !tiled));
     // FLOP-equivalents from the step counts: n * (37 + 25 N_it) per (item, r)
     auto count_flops = [&]() {
         double fl = 0.;
@@ -965,7 +967,6 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
                     ra.flops = b.d_flops;
                     launch_rmarg(g_stream, ra);
                 }
-                copy_out();
                 if (!hip_ok(hipGetLastError(), "likelihood launch") || !q_ok) return false;
                 if (!hip_ok(hipStreamSynchronize(g_stream), "likelihood sync")) return false;
                 if (b.h_status[0] != 0) {  // a task left unfinished: a wait gave up
@@ -982,18 +983,19 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
         if (fused && tuning().fuse_step == 1 && tg[0].tab_y_lds && min_chunks &&
             most_chunks <= kTaskChunks && !tuning().tile_passes && !tuning().tile_blocks &&
             !tuning().tile_cells && tuning().p0_tasks == Tuning().p0_tasks) {
-            want_detail = want_detail || g_stats_on;  // the step counts for the FLOPs
+            if (g_stats_on) want_detail(true);  // the step counts for the FLOPs
+            a.tasks = nullptr;                  // every task ends in the launch
+            TileLaunch t = tg[0];
+            t.lk = a;
+            t.arrived = b.d_arrived;
             {
                 KTimer k(RL2_K_LIKELIHOOD);
-                launch_lik_task(g_stream, tg[0], most_chunks);
+                launch_lik_task(g_stream, t, most_chunks);
             }
-            {
+            if (t.grid != 2) {
                 KTimer k(RL2_K_RMARG);
-                LikLaunch ra = a;
-                ra.tasks = nullptr;  // every task has ended
-                launch_rmarg(g_stream, ra);
+                launch_rmarg(g_stream, a);
             }
-            copy_out();
             if (!hip_ok(hipGetLastError(), "likelihood launch") || !q_ok) return false;
             if (!hip_ok(hipStreamSynchronize(g_stream), "likelihood sync")) return false;
             if (g_stats_on) count_flops();
@@ -1046,7 +1048,6 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
                     ra.flops = b.d_flops;
                     launch_rmarg(g_stream, ra);
                 }
-                copy_out();
                 if (!hip_ok(hipGetLastError(), "likelihood launch") || !q_ok) return false;
                 if (!hip_ok(hipStreamSynchronize(g_stream), "likelihood sync")) return false;
                 if (b.h_status[0] == 0) break;
@@ -1078,7 +1079,6 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
                 ra.flops = b.d_flops;
                 launch_rmarg(g_stream, ra);
             }
-            copy_out();
             if (!hip_ok(hipGetLastError(), "likelihood launch") || !q_ok) return false;
             if (!hip_ok(hipStreamSynchronize(g_stream), "likelihood sync")) return false;
             if (b.h_status[0] == 0) break;
@@ -1104,7 +1104,6 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
             launch_rmarg(g_stream, a);
         }
         if (!hip_ok(hipGetLastError(), "likelihood launch")) return false;
-        copy_out();
         if (!q_ok || !hip_ok(hipStreamSynchronize(g_stream), "likelihood sync")) return false;
         if (g_stats_on) count_flops();
     }
