@@ -120,6 +120,7 @@ Obs *facet_context(size_t n_needed)
         h->o.fmax = f;
         h->o.len = 1.;
         h->o.rg.numr = rl2_r_grid(h->o.rg.ro);
+        rgrid_factor(h->o.rg);
         g_fctx.reset(h);
     }
     return &g_fctx->o;
@@ -136,6 +137,7 @@ bool set_grid(Obs &o, int numr, const double *ro)
     }
     o.rg.numr = numr;
     for (int k = 0; k < kMaxR; k++) o.rg.ro[k] = (k < numr) ? ro[k] : 0.;
+    rgrid_factor(o.rg);
     return true;
 }
 

@@ -55,9 +55,34 @@ struct LikItem {
 
 struct RGrid {
     int numr;                  // 24: ro[1..23] are the models (RadioLensfit2.cpp:370-392)
-    int pad;
+    int factored = 0;          // 1: the arrays below are filled (rgrid_factor)
     double ro[kMaxR];
+    // LDL^T factors of the natural spline's system over the knots ro[1..numr-1], and
+    // 1 / (ro[i + 2] - ro[i + 1]), with spline_init_ws's expressions: they depend on the grid
+    // alone, and almost every evaluation's knots are the whole grid.
+    double alp[kMaxR], gam[kMaxR], ginv[kMaxR];
 };
+// Fills the factors when the grid is one that the spline takes (increasing, at least three
+// inner knots, no zero pivot).
+inline void rgrid_factor(RGrid &g)
+{
+    const int n = g.numr - 1, sys = n - 2;
+    g.factored = 0;
+    for (int i = 0; i < kMaxR; i++) g.alp[i] = g.gam[i] = g.ginv[i] = 0.;
+    if (g.numr > kMaxR || sys < 3) return;
+    const double *x = g.ro + 1;
+    for (int i = 1; i < n; i++)
+        if (!(x[i - 1] < x[i])) return;
+    for (int i = 0; i + 1 < n; i++) g.ginv[i] = 1.0 / (x[i + 1] - x[i]);
+    for (int i = 0; i < sys; i++) {
+        const double h_i = x[i + 1] - x[i], h_ip1 = x[i + 2] - x[i + 1];
+        const double diag = 2.0 * (h_ip1 + h_i);
+        g.alp[i] = i == 0 ? diag : diag - h_i * g.gam[i - 1];  // off_{i-1} = h_i
+        if (g.alp[i] == 0) return;
+        if (i < sys - 1) g.gam[i] = h_ip1 / g.alp[i];
+    }
+    g.factored = 1;
+}
 
 // Streaming-kernel arguments (one galaxy).
 struct GalaxyGeom {

@@ -1074,40 +1074,6 @@ __device__ inline void block_allreduce(double (&v)[N], double *lds)
     __syncthreads();
 }
 
-// Sum of v over the 64 lanes of a wave, in lane 63, by data-parallel-primitive moves (VALU
-// lane shifts, no LDS round trips): shifts by 1, 2, 4 and 8 within each row of 16 lanes
-// leave each row's total in its lane 15; row_bcast:15 adds row 0's total into row 1 and
-// row 2's into row 3, row_bcast:31 adds lane 31's into rows 2 and 3.  Lanes whose source
-// lies outside the row or is masked off add 0.  A fixed order, so the sum is deterministic.
-template <int CTRL, int ROW_MASK, int BANK_MASK>
-__device__ inline double dpp_f64(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    const int rlo = __builtin_amdgcn_update_dpp(0, lo, CTRL, ROW_MASK, BANK_MASK, false);
-    const int rhi = __builtin_amdgcn_update_dpp(0, hi, CTRL, ROW_MASK, BANK_MASK, false);
-    return __hiloint2double(rhi, rlo);
-}
-__device__ inline double wave_sum_last(double v)
-{
-    v += dpp_f64<0x111, 0xf, 0xf>(v);  // row_shr:1
-    v += dpp_f64<0x112, 0xf, 0xf>(v);  // row_shr:2
-    v += dpp_f64<0x114, 0xf, 0xf>(v);  // row_shr:4
-    v += dpp_f64<0x118, 0xf, 0xf>(v);  // row_shr:8
-    v += dpp_f64<0x142, 0xa, 0xf>(v);  // row_bcast:15 into rows 1 and 3
-    v += dpp_f64<0x143, 0xc, 0xf>(v);  // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
-// The wave's sum in every lane: wave_sum_last, then lane 63's value read into scalar
-// registers (every lane gets the same value, so the wave takes the same branches after it).
-__device__ inline double wave_sum(double v)
-{
-    v = wave_sum_last(v);
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
-    return __hiloint2double(hi, lo);
-}
-
 // Lane values read into scalar registers (l uniform over the wave).
 __device__ inline double read_lane(double v, int l)
 {
@@ -1170,11 +1136,22 @@ __device__ inline double wave_sum_by8(double v)
     return v + w;
 }
 
+// The wave's sum in every lane, by data-parallel-primitive moves (lane shifts in the VALU, no
+// LDS round trips): the lanes are paired by bit 0 of their number, then bit 1, and so on, a
+// fixed order, and both lanes of a pair get the same bits.  Read into scalar registers, so
+// that the wave takes the same branches after it.
+__device__ inline double wave_sum(double v)
+{
+    v += dpp_perm_f64<0xb1>(v);  // quad_perm [1, 0, 3, 2]
+    v += dpp_perm_f64<0x4e>(v);  // quad_perm [2, 3, 0, 1]
+    v += dpp_xor4_f64(v);
+    return read_lane(wave_sum_by8(v), 0);
+}
+
 // The wave's sums of eight values at once: the total of v[lane % 8] in every lane.  The lanes
-// are paired by bit 0 of their number, then bit 1, and so on, which is the order in which
-// wave_sum_last adds them (the same bits), but each of the first three steps also halves the
+// are paired as in wave_sum (the same bits), but each of the first three steps also halves the
 // number of values that a lane holds: 10 additions with their moves instead of 48.  The seven
-// sums of a work-group by wave_sum_last took 900 cycles of a Newton pass of 5,700, and those
+// sums of a work-group one after the other took 900 cycles of a Newton pass of 5,700, and those
 // of the task's chunks as much again; with this the loop over 24 galaxies of a 64-dish array
 // went from 26.3 to 24.7 ms, batches of 16 (48 galaxies) from 15.1 to 10.5 ms, 63 points on 496
 // cells from 70.8 to 57.1 us, and 4 points on 72,000 cells from 100.5 to 97.0 us.
@@ -1196,29 +1173,20 @@ __device__ inline double wave_sum8(const double (&v)[8])
     return wave_sum_by8(keep + dpp_xor4_f64(lane & 4 ? x[0] : x[1]));
 }
 
-// The wave's maximum (MAX) or minimum in every lane, by the lane shifts of wave_sum_last; a
-// lane whose source lies outside its row, or in a row masked off, keeps its own value, which
-// leaves the extreme unchanged.  fmax and fmin are exact (and skip NaN), so the result does
-// not depend on the order.
-template <int CTRL, int ROW_MASK>
-__device__ inline double dpp_keep_f64(double v)
+// The wave's maximum in every lane, paired as in wave_sum.  fmax is exact (and skips NaN), so
+// the result does not depend on the order.
+__device__ inline double wave_max(double v)
 {
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    const int rlo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROW_MASK, 0xf, false);
-    const int rhi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROW_MASK, 0xf, false);
-    return __hiloint2double(rhi, rlo);
-}
-template <bool MAX>
-__device__ inline double wave_extreme(double v)
-{
-    auto op = [](double p, double q) { return MAX ? fmax(p, q) : fmin(p, q); };
-    v = op(v, dpp_keep_f64<0x111, 0xf>(v));  // row_shr:1
-    v = op(v, dpp_keep_f64<0x112, 0xf>(v));  // row_shr:2
-    v = op(v, dpp_keep_f64<0x114, 0xf>(v));  // row_shr:4
-    v = op(v, dpp_keep_f64<0x118, 0xf>(v));  // row_shr:8
-    v = op(v, dpp_keep_f64<0x142, 0xa>(v));  // row_bcast:15 into rows 1 and 3
-    v = op(v, dpp_keep_f64<0x143, 0xc>(v));  // row_bcast:31 into rows 2 and 3
-    return read_lane(v, 63);
+    v = fmax(v, dpp_perm_f64<0xb1>(v));
+    v = fmax(v, dpp_perm_f64<0x4e>(v));
+    v = fmax(v, dpp_xor4_f64(v));
+    v = fmax(v, dpp_perm_f64<0x128>(v));
+    double w = v;
+    swap16(v, w);
+    v = fmax(v, w);
+    w = v;
+    swap32(v, w);
+    return read_lane(fmax(v, w), 0);
 }
 
 // expint_ei (rl2_math.h) of two arguments by one wave, the same bits: the divisions of up to 64
@@ -1233,7 +1201,7 @@ __device__ inline void expint_ei_wave(double x0, double x1, double *y0, double *
 {
     const double euler = 0.57721566490153286060651209008240243;
     constexpr int U = 8;
-    __shared__ double buf[2][64];
+    __shared__ double buf[2][64 + U];
     const int lane = threadIdx.x & 63;
     const bool as0 = !(x0 <= 40.), as1 = !(x1 <= 40.);  // asymptotic series
     const double *mine = buf[lane & 1];
@@ -1241,17 +1209,23 @@ __device__ inline void expint_ei_wave(double x0, double x1, double *y0, double *
     // the recurrences over buf[0] and buf[1] in place, by lanes 0 and 1: c = op(c, buf[i])
     auto chain = [&](int steps, double c, auto op) {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        if (lane < 2)
-            for (int i = 0; i < steps; i += U) {
-                double v[U];
+        if (lane < 2) {
+            double v[U], w[U];
 #pragma unroll
-                for (int j = 0; j < U; j++) v[j] = mine[i + j];
+            for (int j = 0; j < U; j++) v[j] = mine[j];
+            for (int i = 0; i < steps; i += U) {
+                // the next values are read before the current ones are used (past the last: the
+                // buffer's tail)
+#pragma unroll
+                for (int j = 0; j < U; j++) w[j] = mine[i + U + j];
 #pragma unroll
                 for (int j = 0; j < U; j++) {
                     c = op(c, v[j]);
                     put[i + j] = c;
+                    v[j] = w[j];
                 }
             }
+        }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         return c;
     };
@@ -1332,7 +1306,9 @@ __device__ inline void finish_lr(const LikLaunch &a, int item, int r, double ho,
             L -= 0.5 * log(det_sigma);
     }
     if ((threadIdx.x & 63) != 0) return;
-    a.Lr[(size_t)item * kMaxR + r] = L;
+    // at agent scope: the small-facet kernel's last work-group of an item reads it
+    __hip_atomic_store(a.Lr + (size_t)item * kMaxR + r, L, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
     a.nit[(size_t)item * kMaxR + r] = iter;
     if (a.Lr_host) {  // pinned memory: the caller reads them after its one synchronisation
         a.Lr_host[(size_t)item * kMaxR + r] = L;
@@ -1946,13 +1922,29 @@ __device__ inline double spline_exp_lds(const SplineLds &t, double x)
     return exp(y);
 }
 
+// What the r-marginalisation reads of an item besides its L_r; a lane holds scalelength index
+// `lane`'s prior and the Gauss-Kronrod node of that number, and row `lane` of the factored
+// spline system of the whole grid.
+struct Gk41Node {
+    double x, wk, wg;
+    int side;  // -1 left, 1 right, 0 the centre (and the unused lanes 41..63)
+};
+struct RmargPre {
+    Gk41Node g;
+    double prior, alp, gam, ginv;
+};
+
 // spline_init_ws (GSL cspline_init semantics) by each wave: lane p holds knot (xp, yp) for
 // p < n, the knots already in t.s.x and t.s.y.  The rows of the tridiagonal system are formed
 // by their lanes at once; the LDL^T recurrences run over lane values read into scalar
 // registers, in spline_init_ws's order and with its expressions, so c, and the b_i and d_i
 // formed from it, are the same bit for bit.  Wave 0 writes n, linear = 0, c, b and d.
+// `whole`: the knots are the whole scalelength grid, whose factorisation (alp, gam and the
+// 1 / h) the host formed once with the same expressions (RGrid): what is left is the two
+// substitutions, 2,500 cycles instead of 8,200, of which 21 dependent divisions were most.
 // Returns spline_init_ws's status, the same in every lane.
-__device__ int spline_build_wave(SplineLds &t, int n, double xp, double yp)
+__device__ int spline_build_wave(SplineLds &t, int n, double xp, double yp, bool whole,
+                                 const RmargPre &pre)
 {
     const int lane = threadIdx.x & 63;
     const bool w0 = threadIdx.x < 64;
@@ -1961,7 +1953,12 @@ __device__ int spline_build_wave(SplineLds &t, int n, double xp, double yp)
     if (__any(lane + 1 < n && !(xp < x1))) return 1;  // knots strictly increasing
     const int max_index = n - 1, sys = max_index - 1;
     double off = 0., diag = 0., g = 0.;
-    if (lane < sys) {
+    const double ginv1 = __shfl_down(pre.ginv, 1);
+    if (whole) {
+        const double yd_i = y1 - yp;
+        const double yd_ip1 = y2 - y1;
+        if (lane < sys) g = 3.0 * (yd_ip1 * ginv1 - yd_i * pre.ginv);
+    } else if (lane < sys) {
         const double h_i = x1 - xp;
         const double h_ip1 = x2 - x1;
         const double yd_i = y1 - yp;
@@ -1977,6 +1974,19 @@ __device__ int spline_build_wave(SplineLds &t, int n, double xp, double yp)
     if (sys == 1) {
         const double c1 = read_lane(g, 0) / read_lane(diag, 0);
         if (lane == 1) c = c1;
+    } else if (whole) {
+        double z = read_lane(g, 0), z_l = z;
+        for (int i = 1; i < sys; i++) {
+            z = read_lane(g, i) - read_lane(pre.gam, i - 1) * z;
+            if (lane == i) z_l = z;
+        }
+        const double cc = lane < sys ? z_l / pre.alp : 0.;
+        double xs = read_lane(cc, sys - 1);
+        if (lane == sys) c = xs;
+        for (int i = sys - 2; i >= 0; i--) {
+            xs = read_lane(cc, i) - read_lane(pre.gam, i) * xs;
+            if (lane == i + 1) c = xs;
+        }
     } else if (sys > 1) {
         // step i: alp_i from gam_{i-1}, the forward substitution's z_i, then gam_i =
         // off_i / alp_i, whose division is the chain's latency; the next step's lane values
@@ -2041,11 +2051,6 @@ __device__ int spline_build_wave(SplineLds &t, int n, double xp, double yp)
 
 // Lane j's Gauss-Kronrod-41 node (0..19 left of the centre, 20..39 right, 40 the centre) and
 // its Kronrod and Gauss weights, read once per work-group.
-struct Gk41Node {
-    double x, wk, wg;
-    int side;  // -1 left, 1 right, 0 the centre (and the unused lanes 41..63)
-};
-
 __device__ inline Gk41Node gk41_node()
 {
     const int lane = threadIdx.x & 63;
@@ -2221,41 +2226,42 @@ __device__ int qag41_wave(const SplineLds &sp, const Gk41Node &g, double a, doub
     return 5;
 }
 
+__device__ inline RmargPre rmarg_pre(const LikLaunch &a, int slot)
+{
+    const int lane = threadIdx.x & 63;
+    const bool mine = lane < kMaxR;
+    RmargPre p;
+    p.g = gk41_node();
+    p.prior = mine ? a.facets[slot].rprior[lane] : 0.;
+    p.alp = mine ? a.rg.alp[lane] : 0.;
+    p.gam = mine ? a.rg.gam[lane] : 0.;
+    p.ginv = mine ? a.rg.ginv[lane] : 0.;
+    return p;
+}
+
 // likelihood.c:126-146 with marginalise_posterior_r (marginalise_r.c:81-223) for one item, by
-// the two waves of the work-group.  Lane r (1 <= r < numR) of each wave reads L_r[r]; the
-// points above kBad go, in r order, to knots 0..num-1 in LDS; ymax, xmin and xmax are wave
-// reductions (xmin and xmax are the extreme abscissae: the reference's start from the
-// neighbours of the maximum does not change them); the QUADPACK lists live in LDS.
-__device__ void rmarg_item(const LikLaunch &a, const LikItem &it, int item, SplineLds &sp,
-                           double *qd, int *qi)
+// the two waves of the work-group.  Lane r (1 <= r < numR) of each wave holds L_r[r] in lv; the
+// points above kBad go, in r order, to knots 0..num-1 in LDS; ymax is a wave reduction; xmin
+// and xmax are the first and the last knot (the extreme abscissae: the reference's start from
+// the neighbours of the maximum does not change them, and knots that do not increase are an
+// error whatever they are); the QUADPACK lists live in LDS.  fragile: a mixed-precision item
+// with a fragile L_r.
+__device__ void rmarg_item(const LikLaunch &a, const RmargPre &pre, double lv, bool fragile,
+                           int item, SplineLds &sp, double *qd, int *qi)
 {
     const int lane = threadIdx.x & 63;
     const int numR = a.rg.numr;
     const bool mine = lane >= 1 && lane < numR;
-    // every global read of the item is issued here, the node tables first
-    const Gk41Node g = gk41_node();
-    const size_t base = (size_t)item * kMaxR;
-    const double lv = mine ? a.Lr[base + lane] : kBad;
-    bool act = false, frag = false;
-    if (a.tasks && mine) {
-        act = a.tasks[base + lane].active;
-        frag = a.tasks[base + lane].fragile;
-    }
-    if (__any(act)) return;  // tiled engine: an item with a task still iterating waits
-    // the node tables have arrived with the loads above: keep them from being re-read later
-    asm volatile("" ::"v"(g.x), "v"(g.wk), "v"(g.wg));
-    const bool fragile = it.prec == 1 && __any(frag);
+    const Gk41Node &g = pre.g;
     const bool ok = mine && lv > kBad;
     const double xr = mine ? a.rg.ro[lane] : 0.;
-    const double yr = ok ? lv + a.facets[it.slot].rprior[lane] : 0.;
+    const double yr = ok ? lv + pre.prior : 0.;
     const uint64_t m = __ballot(ok);
     const int num = __popcll(m);
     int error = 0;
     double L_e;
     if (num > 4) {
-        const double ymax = wave_extreme<true>(ok && yr > -10.0 ? yr : -10.0);
-        const double xmin = wave_extreme<false>(ok ? xr : INFINITY);
-        const double xmax = wave_extreme<true>(ok ? xr : -INFINITY);
+        const double ymax = wave_max(ok && yr > -10.0 ? yr : -10.0);
         const int pos = __popcll(m & ((1ull << lane) - 1ull));
         if (threadIdx.x < 64 && ok) {
             sp.s.x[pos] = xr;
@@ -2264,7 +2270,9 @@ __device__ void rmarg_item(const LikLaunch &a, const LikItem &it, int item, Spli
         __syncthreads();
         const double xp = lane < num ? sp.s.x[lane] : 0.;
         const double yp = lane < num ? sp.s.y[lane] : 0.;
-        if (xmax <= xmin || spline_build_wave(sp, num, xp, yp)) {
+        const double xmin = read_lane(xp, 0), xmax = read_lane(xp, num - 1);
+        if (xmax <= xmin ||
+            spline_build_wave(sp, num, xp, yp, a.rg.factored && num == numR - 1, pre)) {
             L_e = NAN;
         } else {
             QagWs w;
@@ -2311,7 +2319,22 @@ __global__ __launch_bounds__(128) void rmarg_kernel(LikLaunch a)
     __shared__ SplineLds sp;
     __shared__ double qd[kQagDoubles];
     __shared__ int qi[kQagInts];
-    rmarg_item(a, a.items[blockIdx.x], blockIdx.x, sp, qd, qi);
+    const LikItem it = a.items[blockIdx.x];
+    const int lane = threadIdx.x & 63;
+    const bool mine = lane >= 1 && lane < a.rg.numr;
+    // every global read of the item is issued here, the node tables first
+    const RmargPre pre = rmarg_pre(a, it.slot);
+    const size_t base = (size_t)blockIdx.x * kMaxR;
+    const double lv = mine ? a.Lr[base + lane] : kBad;
+    bool act = false, frag = false;
+    if (a.tasks && mine) {
+        act = a.tasks[base + lane].active;
+        frag = a.tasks[base + lane].fragile;
+    }
+    if (__any(act)) return;  // tiled engine: an item with a task still iterating waits
+    // the node tables have arrived with the loads above: keep them from being re-read later
+    asm volatile("" ::"v"(pre.g.x), "v"(pre.g.wk), "v"(pre.g.wg));
+    rmarg_item(a, pre, lv, it.prec == 1 && __any(frag), blockIdx.x, sp, qd, qi);
 }
 
 // ------------------------------------------------------------------ likelihood, tiled
@@ -3913,14 +3936,21 @@ __global__ __launch_bounds__(kTileBS *G, NC == 1 ? 3 : 2) void lik_task_kernel(T
             put(k, s);
         }
     }
-    if (threadIdx.x < 64) finish_lr(a, item, r, ho, det, S.iter);
-    if constexpr (KIND == 2) {
+    if constexpr (KIND != 2) {
+        if (threadIdx.x < 64) finish_lr(a, item, r, ho, det, S.iter);
+    } else {
         __shared__ SplineLds sp;
         __shared__ bool s_last;
         if (threadIdx.x >= 128) return;
+        // in flight while the task ends: what the integral reads besides the L_r
+        const RmargPre pre = rmarg_pre(a, it.slot);
+        asm volatile("" ::"v"(pre.g.x), "v"(pre.g.wk), "v"(pre.g.wg));
+        if (threadIdx.x < 64) finish_lr(a, item, r, ho, det, S.iter);
         if (threadIdx.x == 0) {
-            // lane 0 wrote L_r: released with this count, and the other tasks' acquired
-            const unsigned k = __hip_atomic_fetch_add(t.arrived + item, 1u, __ATOMIC_ACQ_REL,
+            // lane 0 stored L_r at agent scope: the store has completed before the count (the
+            // fences of a release and an acquire write back and drop the XCD's whole L2)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            const unsigned k = __hip_atomic_fetch_add(t.arrived + item, 1u, __ATOMIC_RELAXED,
                                                       __HIP_MEMORY_SCOPE_AGENT);
             s_last = k + 1 == (unsigned)t.nr_g;
             if (s_last)  // zero again for the next launch
@@ -3929,8 +3959,12 @@ __global__ __launch_bounds__(kTileBS *G, NC == 1 ? 3 : 2) void lik_task_kernel(T
         }
         __syncthreads();
         if (!s_last) return;
+        const double lv = lane >= 1 && lane < a.rg.numr
+                              ? __hip_atomic_load(a.Lr + (size_t)item * kMaxR + lane,
+                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                              : kBad;
         double *qd = reinterpret_cast<double *>(tab_lds);  // the records are done with
-        rmarg_item(a, it, item, sp, qd, reinterpret_cast<int *>(qd + kQagDoubles));
+        rmarg_item(a, pre, lv, false, item, sp, qd, reinterpret_cast<int *>(qd + kQagDoubles));
     }
 }
 

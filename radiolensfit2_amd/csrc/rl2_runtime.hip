@@ -1468,6 +1468,7 @@ int rl2_obs_create(rl2_obs **out, unsigned int nch, unsigned long nrow, const do
     o.fmax = facet_size(kRmax, len);
     o.rg.numr = rl2_r_grid(o.rg.ro);
     for (int k = o.rg.numr; k < kMaxR; k++) o.rg.ro[k] = 0.;
+    rgrid_factor(o.rg);
     o.wn.assign(wavenumbers, wavenumbers + nch);
     o.spec.assign(spec, spec + nch);
     o.invlam.resize(nch);
@@ -1769,6 +1770,7 @@ int rl2_rmarg_eval(int nitems, int numr, const double *ro, const double *rprior,
         a.facets = d_f;
         a.rg.numr = numr;
         for (int k = 0; k < kMaxR; k++) a.rg.ro[k] = k < numr ? ro[k] : 0.;
+        rgrid_factor(a.rg);
         a.Lr = d_Lr;
         a.Le = d_Le;
         a.err = d_err;
