@@ -1112,6 +1112,17 @@ __device__ inline double dpp_perm_f64(double v)
     return __hiloint2double(rhi, rlo);
 }
 
+// Shifts over the whole wave by one lane (0x138 wave_shr:1: from the lane before, 0x130
+// wave_shl:1: from the lane after); 0 where there is none.
+template <int CTRL>
+__device__ inline double dpp_shift_f64(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    const int rlo = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, true);
+    const int rhi = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, true);
+    return __hiloint2double(rhi, rlo);
+}
+
 // Each lane's value of the lane whose number differs in bit 2 (the other half of its eight):
 // shifts by 4 into the banks of four lanes that have a source in their half.
 __device__ inline double dpp_xor4_f64(double v)
@@ -1210,20 +1221,26 @@ __device__ inline void expint_ei_wave(double x0, double x1, double *y0, double *
     auto chain = [&](int steps, double c, auto op) {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         if (lane < 2) {
+            // two sets of U values, each read while the other is used (past the last: the
+            // buffer's tail); no copies between them, which would wait for the reads
             double v[U], w[U];
-#pragma unroll
-            for (int j = 0; j < U; j++) v[j] = mine[j];
-            for (int i = 0; i < steps; i += U) {
-                // the next values are read before the current ones are used (past the last: the
-                // buffer's tail)
-#pragma unroll
-                for (int j = 0; j < U; j++) w[j] = mine[i + U + j];
+            auto use = [&](const double (&x)[U], int i) {
 #pragma unroll
                 for (int j = 0; j < U; j++) {
-                    c = op(c, v[j]);
+                    c = op(c, x[j]);
                     put[i + j] = c;
-                    v[j] = w[j];
                 }
+            };
+            auto read = [&](double (&x)[U], int i) {
+#pragma unroll
+                for (int j = 0; j < U; j++) x[j] = mine[i + j];
+            };
+            read(v, 0);
+            for (int i = 0; i < steps; i += 2 * U) {
+                read(w, i + U);
+                use(v, i);
+                read(v, i + 2 * U);
+                use(w, i + U);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1233,7 +1250,8 @@ __device__ inline void expint_ei_wave(double x0, double x1, double *y0, double *
     double s0 = 0., s1 = 0.;
     bool done0 = false, done1 = false;
     for (int base = 0; base < 1024 && !(done0 && done1); base += 64) {
-        const int steps = min(64, ((int)(2.2 * fmin(fmax(x0, x1), 40.)) + 24 + U - 1) / U * U);
+        const int steps =
+            min(64, ((int)(2.2 * fmin(fmax(x0, x1), 40.)) + 24 + 2 * U - 1) / (2 * U) * (2 * U));
         const double k = (double)(base + lane + 1);
         buf[0][lane] = as0 ? k / x0 : x0 / k;
         buf[1][lane] = as1 ? k / x1 : x1 / k;
@@ -1941,7 +1959,9 @@ struct RmargPre {
 // formed from it, are the same bit for bit.  Wave 0 writes n, linear = 0, c, b and d.
 // `whole`: the knots are the whole scalelength grid, whose factorisation (alp, gam and the
 // 1 / h) the host formed once with the same expressions (RGrid): what is left is the two
-// substitutions, 2,500 cycles instead of 8,200, of which 21 dependent divisions were most.
+// substitutions, without the 21 dependent divisions.  With the series' read-ahead
+// (expint_ei_wave) an evaluation of a 64-dish loop took the small-facet kernel 17.4 us
+// instead of 19.9, and the kernel of many items 9.9 instead of 12.1.
 // Returns spline_init_ws's status, the same in every lane.
 __device__ int spline_build_wave(SplineLds &t, int n, double xp, double yp, bool whole,
                                  const RmargPre &pre)
@@ -1975,18 +1995,17 @@ __device__ int spline_build_wave(SplineLds &t, int n, double xp, double yp, bool
         const double c1 = read_lane(g, 0) / read_lane(diag, 0);
         if (lane == 1) c = c1;
     } else if (whole) {
-        double z = read_lane(g, 0), z_l = z;
-        for (int i = 1; i < sys; i++) {
-            z = read_lane(g, i) - read_lane(pre.gam, i - 1) * z;
-            if (lane == i) z_l = z;
-        }
-        const double cc = lane < sys ? z_l / pre.alp : 0.;
-        double xs = read_lane(cc, sys - 1);
-        if (lane == sys) c = xs;
-        for (int i = sys - 2; i >= 0; i--) {
-            xs = read_lane(cc, i) - read_lane(pre.gam, i) * xs;
-            if (lane == i + 1) c = xs;
-        }
+        // every lane takes its row's step again and again from its neighbour's value: lane i
+        // has its final value after i steps and keeps it
+        const double gam1 = dpp_shift_f64<0x138>(pre.gam);  // lane i: gam_{i-1} (lane 0: 0)
+        double z = g;
+        for (int i = 1; i < sys; i++) z = g - gam1 * dpp_shift_f64<0x138>(z);
+        const double cc = lane < sys ? z / pre.alp : 0.;
+        const double gm = lane < sys - 1 ? pre.gam : 0.;
+        double xs = cc;
+        for (int i = 1; i < sys; i++) xs = cc - gm * dpp_shift_f64<0x130>(xs);
+        xs = dpp_shift_f64<0x138>(xs);  // c_{i+1} = x_i
+        if (lane >= 1 && lane <= sys) c = xs;
     } else if (sys > 1) {
         // step i: alp_i from gam_{i-1}, the forward substitution's z_i, then gam_i =
         // off_i / alp_i, whose division is the chain's latency; the next step's lane values
