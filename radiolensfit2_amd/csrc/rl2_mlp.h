@@ -28,10 +28,10 @@ struct MlpGemm {
     const float *bias;  // optional, per column n
     float *pre;         // optional: pre-activation copy (same strides as C)
     int act;            // 1: GELU
+    const float *back = nullptr;  // optional: times gelu'(back), at C's place
+    float *db = nullptr;          // optional: db[m] = sum_k A(m, k), in FP32 in the order of k
 };
 void launch_mlp_gemm(hipStream_t s, const MlpGemm &g);
-void launch_mlp_gelu_back(hipStream_t s, long n, const float *pre, const float *dout, float *dpre);
-void launch_mlp_bias_grad(hipStream_t s, int B, int N, const float *dY, float *db);
 void launch_mlp_nll(hipStream_t s, int B, const float *out, const float *y, float *dout,
                     float *loss);
 void launch_mlp_adam(hipStream_t s, long n, float *p, const float *g, float *m, float *v,
@@ -58,7 +58,7 @@ struct Mlp {
     float *x = nullptr;                       // cap * In
     float *act[kMlpLayers] = {};              // outputs of each layer, cap * n_out
     float *pre[kMlpLayers] = {};              // pre-activations
-    float *dact = nullptr, *dpre = nullptr;   // cap * max width
+    float *dact = nullptr, *dpre = nullptr;   // cap * max width, in turn by layer
     float *y = nullptr, *loss = nullptr;      // cap * 3, cap
     float *h_loss = nullptr;                  // pinned, cap
     ~Mlp();

@@ -32,71 +32,145 @@ __device__ inline float gelu_grad(float x)
 
 // C[m][n] = sum_k A(m, k) B(k, n) (+ bias[n]) with A(m, k) = A[m*sam + k*sak] and
 // B(k, n) = B[k*sbk + n*sbn]; operands rounded to BF16, products accumulated in FP32 by
-// v_mfma_f32_16x16x16_bf16.  One wave per 16x16 tile of C, four waves per work-group.
+// v_mfma_f32_16x16x16_bf16, in the order of k.
 // MFMA 16x16x16 operand layout: lane l supplies A row l%16, k = 4(l/16)..4(l/16)+3 and B
 // column l%16, the same k; it receives C rows 4(l/16)..+3 of column l%16.
-__global__ __launch_bounds__(256) void mlp_gemm_kernel(MlpGemm g)
-{
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int ntn = (g.N + 15) / 16, ntm = (g.M + 15) / 16;
-    const int tile = blockIdx.x * 4 + wave;
-    if (tile >= ntm * ntn) return;
-    const int tm = tile / ntn, tn = tile % ntn;
-    const int r16 = lane & 15, kq = (lane >> 4) * 4;
-    const int arow = tm * 16 + r16, bcol = tn * 16 + r16;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < g.K; k0 += 16) {
-        bf16x4 a, b;
+// One work-group per 16x16 tile of C: the products are few (a batch of 256 has 65k to 51M a
+// layer) and the time is memory latency, so all four waves fetch, convert and stage kGemmK
+// values of k of both operands in LDS in one go (512 of them: two rounds at K = 770), and
+// wave 0 multiplies.  For a batch of 256 a wave per tile that fetched 16 values of k, waited
+// and multiplied took 15.4 us a product; this takes 7 to 10.  With the activation's gradient in
+// the product's epilogue and the bias gradients in the weight gradients' launch (they took 23 us
+// each on one work-group) loss and gradient went from 420 to 242 us, copies included.
+// Staged as [k / 4][row] groups of four k: a wave's operand reads are 512 consecutive bytes.
+constexpr int kGemmK = 512;
+
+// 16 rows (columns of B) of an operand from r0, and where thread t's four values of k go in
+// the staged block of k from k0.  KFAST: consecutive lanes along k (a row's values are adjacent
+// in memory), else along the rows.
+template <bool KFAST>
+struct GemmOperand {
+    const float *P;
+    long sr, sk;
+    int r0, nr;
+    __device__ int slot(int t) const
+    {
+        return KFAST ? ((t & 15) + (t >> 8) * 16) * 16 + ((t >> 4) & 15) : t;
+    }
+    __device__ void fetch(float (&f)[4], int t, int k0, int kend) const
+    {
+        const int s = slot(t), k4 = k0 + 4 * (s >> 4), r = r0 + (s & 15);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int k = k0 + kq + i;
-            const float av = (arow < g.M && k < g.K) ? g.A[(long)arow * g.sam + (long)k * g.sak] : 0.f;
-            const float bv = (bcol < g.N && k < g.K) ? g.B[(long)k * g.sbk + (long)bcol * g.sbn] : 0.f;
-            a[i] = to_bf16(av);
-            b[i] = to_bf16(bv);
+            const bool in = r < nr && k4 + i < kend;
+            f[i] = in ? P[(long)r * sr + (long)(k4 + i) * sk] : 0.f;
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
     }
+    __device__ void put(bf16x4 *lds, const float (&f)[4], int t, int groups) const
+    {
+        const int s = slot(t);
+        if ((s >> 4) >= groups) return;
+        bf16x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = to_bf16(f[i]);
+        lds[s] = v;
+    }
+};
+
+// db[j] = sum_b dY[b][j], added in the order of b: 32 columns a work-group, whose threads
+// fetch 256 rows at a time.
+constexpr int kBiasCols = 32, kBiasRows = 256;
+__device__ inline void gemm_bias_grad(const MlpGemm &g, int j0, float *lds)
+{
+    const int col = threadIdx.x & (kBiasCols - 1), j = j0 + col;
+    float s = 0.f;
+    for (int b0 = 0; b0 < g.K; b0 += kBiasRows) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kBiasCols; i++) {
+            const int r = i * (256 / kBiasCols) + (int)threadIdx.x / kBiasCols;
+            lds[r * kBiasCols + col] =
+                b0 + r < g.K && j < g.M ? g.A[(long)j * g.sam + (long)(b0 + r) * g.sak] : 0.f;
+        }
+        __syncthreads();
+        const int n = min(kBiasRows, g.K - b0);
+        if (threadIdx.x < kBiasCols) {
+#pragma unroll 8
+            for (int r = 0; r < n; r++) s += lds[r * kBiasCols + col];
+        }
+    }
+    if (threadIdx.x < kBiasCols && j < g.M) g.db[j] = s;
+}
+
+template <bool AK, bool BK>
+__global__ __launch_bounds__(256) void mlp_gemm_kernel(MlpGemm g)
+{
+    __shared__ bf16x4 lds[2 * kGemmK / 4 * 16];
+    static_assert(sizeof(lds) >= kBiasCols * kBiasRows * sizeof(float), "bias rows");
+    bf16x4 *sA = lds, *sB = lds + kGemmK / 4 * 16;
+    const int lane = threadIdx.x & 63;
+    const int ntn = (g.N + 15) / 16, ntm = (g.M + 15) / 16;
+    const int tile = blockIdx.x;
+    if (tile >= ntm * ntn) {  // the blocks after the tiles: the bias gradient
+        gemm_bias_grad(g, (tile - ntm * ntn) * kBiasCols, reinterpret_cast<float *>(lds));
+        return;
+    }
+    const int tm = tile / ntn, tn = tile % ntn;
+    const GemmOperand<AK> opA{g.A, g.sam, g.sak, tm * 16, g.M};
+    const GemmOperand<BK> opB{g.B, g.sbn, g.sbk, tn * 16, g.N};
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < g.K; k0 += kGemmK) {
+        if (k0) __syncthreads();
+        // the last step of 16 may reach past the staged groups
+        const int kn = min(kGemmK, g.K - k0), groups = (kn + 3) / 4, need = (kn + 15) / 16 * 4;
+        constexpr int U = 4;  // four groups of each operand in flight per thread: K = 256
+        for (int t = threadIdx.x; t < (groups + 15) / 16 * 256; t += 256 * U) {
+            float fa[U][4], fb[U][4];
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                opA.fetch(fa[q], t + 256 * q, k0, g.K);
+                opB.fetch(fb[q], t + 256 * q, k0, g.K);
+            }
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                opA.put(sA, fa[q], t + 256 * q, groups);
+                opB.put(sB, fb[q], t + 256 * q, groups);
+            }
+        }
+        if ((int)threadIdx.x < (need - groups) * 16) {
+            sA[groups * 16 + threadIdx.x] = bf16x4{0, 0, 0, 0};
+            sB[groups * 16 + threadIdx.x] = bf16x4{0, 0, 0, 0};
+        }
+        __syncthreads();
+        if (threadIdx.x < 64)
+            for (int k = 0; k < need * 16; k += 64)
+                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(sA[k + lane], sB[k + lane], acc, 0,
+                                                                0, 0);
+    }
+    if (threadIdx.x >= 64) return;
+    const int kq = (lane >> 4) * 4, c = tn * 16 + (lane & 15);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const int r = tm * 16 + kq + i, c = bcol;
+        const int r = tm * 16 + kq + i;
         if (r >= g.M || c >= g.N) continue;
+        const long at = (long)r * g.scm + (long)c * g.scn;
         float x = acc[i] + (g.bias ? g.bias[c] : 0.f);
-        if (g.pre) g.pre[(long)r * g.scm + (long)c * g.scn] = x;
+        if (g.pre) g.pre[at] = x;
         if (g.act) x = gelu(x);
-        g.C[(long)r * g.scm + (long)c * g.scn] = x;
+        if (g.back) x *= gelu_grad(g.back[at]);
+        g.C[at] = x;
     }
 }
 
 void launch_mlp_gemm(hipStream_t s, const MlpGemm &g)
 {
-    const int tiles = ((g.M + 15) / 16) * ((g.N + 15) / 16);
-    mlp_gemm_kernel<<<(tiles + 3) / 4, 256, 0, s>>>(g);
-}
-
-// d_pre = d_out * gelu'(pre)
-__global__ void mlp_gelu_back_kernel(long n, const float *pre, const float *dout, float *dpre)
-{
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-        dpre[i] = dout[i] * gelu_grad(pre[i]);
-}
-void launch_mlp_gelu_back(hipStream_t s, long n, const float *pre, const float *dout, float *dpre)
-{
-    mlp_gelu_back_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, pre, dout, dpre);
-}
-
-// db[j] = sum_b dY[b][j]
-__global__ void mlp_bias_grad_kernel(int B, int N, const float *dY, float *db)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= N) return;
-    float s = 0.f;
-    for (int b = 0; b < B; b++) s += dY[(long)b * N + j];
-    db[j] = s;
-}
-void launch_mlp_bias_grad(hipStream_t s, int B, int N, const float *dY, float *db)
-{
-    mlp_bias_grad_kernel<<<(N + 255) / 256, 256, 0, s>>>(B, N, dY, db);
+    const int blocks = ((g.M + 15) / 16) * ((g.N + 15) / 16) + (g.db ? (g.M + kBiasCols - 1) / kBiasCols : 0);
+    if (g.sak == 1 && g.sbk == 1)
+        mlp_gemm_kernel<true, true><<<blocks, 256, 0, s>>>(g);
+    else if (g.sak == 1)
+        mlp_gemm_kernel<true, false><<<blocks, 256, 0, s>>>(g);
+    else
+        mlp_gemm_kernel<false, false><<<blocks, 256, 0, s>>>(g);
 }
 
 // Gaussian negative log-likelihood of the target y = (e1, e2, log r) under the output

@@ -4,6 +4,7 @@
 #include <math.h>
 #include <stdint.h>
 #include <string.h>
+#include <utility>
 #include <vector>
 
 #include "rl2_mlp.h"
@@ -118,15 +119,16 @@ bool Mlp::forward(hipStream_t s, int B)
 bool Mlp::backward(hipStream_t s, int B)
 {
     launch_mlp_nll(s, B, act[kMlpLayers - 1], y, dpre, loss);
+    float *d = dpre, *dn = dact;  // this layer's d loss / d pre, and the next one's
     for (int l = kMlpLayers - 1; l >= 0; l--) {
         const int in = mlp_in(l), out = mlp_out(l);
         const float *xin = l == 0 ? x : act[l - 1];
-        // dW = dpre^T x
+        // dW = d^T x, and db = the column sums of d
         MlpGemm gw;
         gw.M = out;
         gw.N = in;
         gw.K = B;
-        gw.A = dpre;
+        gw.A = d;
         gw.sam = 1;
         gw.sak = out;
         gw.B = xin;
@@ -138,28 +140,29 @@ bool Mlp::backward(hipStream_t s, int B)
         gw.bias = nullptr;
         gw.pre = nullptr;
         gw.act = 0;
+        gw.db = g + mlp_b_off(l);
         launch_mlp_gemm(s, gw);
-        launch_mlp_bias_grad(s, B, out, dpre, g + mlp_b_off(l));
         if (l == 0) break;
-        // dact = dpre W ; dpre(l-1) = dact * gelu'(pre(l-1))
+        // d of the layer before: (d W) gelu'(pre(l-1))
         MlpGemm gx;
         gx.M = B;
         gx.N = in;
         gx.K = out;
-        gx.A = dpre;
+        gx.A = d;
         gx.sam = out;
         gx.sak = 1;
         gx.B = p + mlp_w_off(l);
         gx.sbk = in;
         gx.sbn = 1;
-        gx.C = dact;
+        gx.C = dn;
         gx.scm = in;
         gx.scn = 1;
         gx.bias = nullptr;
         gx.pre = nullptr;
         gx.act = 0;
+        gx.back = pre[l - 1];
         launch_mlp_gemm(s, gx);
-        launch_mlp_gelu_back(s, (long)B * in, pre[l - 1], dact, dpre);
+        std::swap(d, dn);
     }
     return hip_ok(hipGetLastError(), "mlp backward");
 }
