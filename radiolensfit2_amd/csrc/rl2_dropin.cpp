@@ -687,19 +687,21 @@ void sky_model(double *wavenumbers, double *spec, double, int, unsigned int num_
     if (!ensure_device()) return;
     const size_t nvis = (size_t)num_channels * num_coords;
     DBuf<double> du(num_coords), dv(num_coords), dw(num_coords), dwn(num_channels),
-        dsp(num_channels), dres(2 * nvis);
+        dil(num_channels), dsp(num_channels), dres(2 * nvis);
     DBuf<GalaxyGeom> dg(n_gal);
     std::vector<GalaxyGeom> g(n_gal);
+    std::vector<double> il(num_channels);
+    for (unsigned c = 0; c < num_channels; c++) il[c] = wavenumbers[c] / (2. * kPi);
     for (unsigned i = 0; i < n_gal; i++) g[i] = make_geom(l[i], m[i], gflux[i], gscale[i], 0., 0.);
-    if (!allocated(du, dv, dw, dwn, dsp, dres, dg) || !du.up(uu_metres, num_coords) ||
+    if (!allocated(du, dv, dw, dwn, dil, dsp, dres, dg) || !du.up(uu_metres, num_coords) ||
         !dv.up(vv_metres, num_coords) || !dw.up(ww_metres, num_coords) ||
-        !dwn.up(wavenumbers, num_channels) || !dsp.up(spec, num_channels) ||
-        !dres.up((const double *)visMod, 2 * nvis) || !dg.up(g.data(), n_gal)) {
+        !dwn.up(wavenumbers, num_channels) || !dil.up(il.data(), num_channels) ||
+        !dsp.up(spec, num_channels) || !dres.up((const double *)visMod, 2 * nvis) || !dg.up(g.data(), n_gal)) {
         report("sky_model");
         return;
     }
-    launch_add_sources(stream(), 0, num_channels, num_coords, du.p, dv.p, dw.p, dwn.p, dsp.p, dg.p,
-                       n_gal, 1.0, dres.p);
+    launch_add_sources(stream(), 0, num_channels, num_coords, du.p, dv.p, dw.p, dwn.p, dil.p,
+                       dsp.p, dg.p, n_gal, 1.0, dres.p);
     if (!dres.down((double *)visMod, 2 * nvis) || !sync_ok()) report("sky_model");
 }
 

@@ -98,8 +98,8 @@ struct GalaxyGeom {
 // R[c][i] += sign * sum_g model_g ; gal: ngal GalaxyGeom on the device.
 void launch_add_sources(hipStream_t s, int prec, unsigned nch, unsigned long nrow,
                         const double *u, const double *v, const double *w, const double *wn,
-                        const double *spec, const GalaxyGeom *gal, unsigned ngal, double sign,
-                        void *res);
+                        const double *inv_lambda, const double *spec, const GalaxyGeom *gal,
+                        unsigned ngal, double sign, void *res);
 void launch_add_noise(hipStream_t s, int prec, unsigned long nvis, double sigma, uint64_t seed,
                       void *res);
 

@@ -84,79 +84,92 @@ __device__ inline double2 subtract_vis(const GalaxyGeom &fit, const GalaxyGeom &
 // ------------------------------------------------------------------ sources / noise
 // R += sign * sum_g flux_g spec_c shape_g exp(i k_c (u l + v m + w n)).
 // One thread per row; galaxies staged through LDS in tiles of 128.
+// Bound by FP64 issue (a phase and a model per galaxy and visibility, 55 FP64 and integer
+// instructions), so the phase goes through sincos_rev64 and the model through one reciprocal
+// square root, and whole blocks of CB channels run without a test per channel.  500 galaxies
+// on 3.87M visibilities: 3.7 ms; 7.3 with the library's sincos and a square root and a division
+// per model (the error against 64 bits, 1.6e-12 of the model on phases of up to 100
+// revolutions, is the phase's own rounding in both).
+template <int PREC, int CB>
+__device__ inline void add_sources_block(const GalaxyGeom *__restrict__ gal, unsigned ngal,
+                                         unsigned c0, unsigned long nrow, unsigned long i,
+                                         double ui, double vi, double wi,
+                                         const double *__restrict__ wn,
+                                         const double *__restrict__ inv_lambda,
+                                         const double *__restrict__ spec, double sign, void *res)
+{
+    constexpr int TILE = 128;
+    __shared__ GalaxyGeom sg[TILE];
+    double are[CB], aim[CB];
+#pragma unroll
+    for (int k = 0; k < CB; k++) are[k] = aim[k] = 0.;
+    for (unsigned g0 = 0; g0 < ngal; g0 += TILE) {
+        __syncthreads();
+        for (unsigned t = threadIdx.x; t < TILE && g0 + t < ngal; t += blockDim.x)
+            sg[t] = gal[g0 + t];
+        __syncthreads();
+        const unsigned gn = min((unsigned)TILE, ngal - g0);
+        for (unsigned t = 0; t < gn; t++) {
+            const GalaxyGeom g = sg[t];
+            const double p = ui * g.l0 + vi * g.m0 + wi * g.n0;
+#pragma unroll
+            for (int k = 0; k < CB; k++) {
+                // the phase k p in revolutions is p / lambda
+                const double wnc = wn[c0 + k];
+                const double shape = model_shape_rsq(g, ui, vi, wnc * wnc, spec[c0 + k]);
+                double sn, cs;
+                sincos_rev64(p * inv_lambda[c0 + k], sn, cs);
+                are[k] = fma(shape, cs, are[k]);
+                aim[k] = fma(shape, sn, aim[k]);
+            }
+        }
+    }
+    if (i >= nrow) return;
+#pragma unroll
+    for (int k = 0; k < CB; k++) {
+        const size_t idx = (size_t)(c0 + k) * nrow + i;
+        double2 r = load_res(res, PREC, idx);
+        r.x += sign * are[k];
+        r.y += sign * aim[k];
+        store_res(res, PREC, idx, r);
+    }
+}
+
 template <int PREC>
 __global__ __launch_bounds__(256) void add_sources_kernel(unsigned nch, unsigned long nrow,
                                                           const double *__restrict__ u,
                                                           const double *__restrict__ v,
                                                           const double *__restrict__ w,
                                                           const double *__restrict__ wn,
+                                                          const double *__restrict__ inv_lambda,
                                                           const double *__restrict__ spec,
                                                           const GalaxyGeom *__restrict__ gal,
                                                           unsigned ngal, double sign, void *res)
 {
-    constexpr int TILE = 128;
-    constexpr int CB = 8;  // channels per register block
-    __shared__ GalaxyGeom sg[TILE];
-    unsigned long i = blockIdx.x * (unsigned long)blockDim.x + threadIdx.x;
-    bool ok = i < nrow;
-    double ui = ok ? u[i] : 0., vi = ok ? v[i] : 0., wi = ok ? w[i] : 0.;
-    for (unsigned c0 = 0; c0 < nch; c0 += CB) {
-        double are[CB], aim[CB], wnc[CB], wn2[CB], spc[CB];
-        int nc = min((int)(nch - c0), CB);
-#pragma unroll
-        for (int k = 0; k < CB; k++) {
-            are[k] = 0.;
-            aim[k] = 0.;
-            wnc[k] = (k < nc) ? wn[c0 + k] : 0.;
-            wn2[k] = wnc[k] * wnc[k];
-            spc[k] = (k < nc) ? spec[c0 + k] : 0.;
-        }
-        for (unsigned g0 = 0; g0 < ngal; g0 += TILE) {
-            __syncthreads();
-            for (unsigned t = threadIdx.x; t < TILE && g0 + t < ngal; t += blockDim.x)
-                sg[t] = gal[g0 + t];
-            __syncthreads();
-            unsigned gn = min((unsigned)TILE, ngal - g0);
-            for (unsigned t = 0; t < gn; t++) {
-                const GalaxyGeom g = sg[t];
-                double p = ui * g.l0 + vi * g.m0 + wi * g.n0;
-#pragma unroll
-                for (int k = 0; k < CB; k++) {
-                    if (k < nc) {
-                        double phase = wnc[k] * p;
-                        double shape = model_shape(g, ui, vi, wn2[k], spc[k]);
-                        double sn, cs;
-                        sincos(phase, &sn, &cs);
-                        are[k] += shape * cs;
-                        aim[k] += shape * sn;
-                    }
-                }
-            }
-        }
-        if (ok) {
-            for (int k = 0; k < nc; k++) {
-                size_t idx = (size_t)(c0 + k) * nrow + i;
-                double2 r = load_res(res, PREC, idx);
-                r.x += sign * are[k];
-                r.y += sign * aim[k];
-                store_res(res, PREC, idx, r);
-            }
-        }
-    }
+    const unsigned long i = blockIdx.x * (unsigned long)blockDim.x + threadIdx.x;
+    const bool ok = i < nrow;
+    const double ui = ok ? u[i] : 0., vi = ok ? v[i] : 0., wi = ok ? w[i] : 0.;
+    unsigned c0 = 0;
+    for (; c0 + 4 <= nch; c0 += 4)
+        add_sources_block<PREC, 4>(gal, ngal, c0, nrow, i, ui, vi, wi, wn, inv_lambda, spec, sign,
+                                   res);
+    for (; c0 < nch; c0++)
+        add_sources_block<PREC, 1>(gal, ngal, c0, nrow, i, ui, vi, wi, wn, inv_lambda, spec, sign,
+                                   res);
 }
 
 void launch_add_sources(hipStream_t s, int prec, unsigned nch, unsigned long nrow,
                         const double *u, const double *v, const double *w, const double *wn,
-                        const double *spec, const GalaxyGeom *gal, unsigned ngal, double sign,
-                        void *res)
+                        const double *inv_lambda, const double *spec, const GalaxyGeom *gal,
+                        unsigned ngal, double sign, void *res)
 {
     dim3 grid((unsigned)((nrow + 255) / 256));
     if (prec == 0)
-        add_sources_kernel<0><<<grid, 256, 0, s>>>(nch, nrow, u, v, w, wn, spec, gal, ngal,
-                                                    sign, res);
+        add_sources_kernel<0><<<grid, 256, 0, s>>>(nch, nrow, u, v, w, wn, inv_lambda, spec, gal,
+                                                    ngal, sign, res);
     else
-        add_sources_kernel<1><<<grid, 256, 0, s>>>(nch, nrow, u, v, w, wn, spec, gal, ngal,
-                                                    sign, res);
+        add_sources_kernel<1><<<grid, 256, 0, s>>>(nch, nrow, u, v, w, wn, inv_lambda, spec, gal,
+                                                    ngal, sign, res);
 }
 
 template <int PREC>
@@ -1008,18 +1021,35 @@ __global__ __launch_bounds__(256) void abs_bound_kernel(const void *res, unsigne
                                                         unsigned long long *out)
 {
     double m = 0.;
-    for (unsigned long i = blockIdx.x * 256ul + threadIdx.x; i < n; i += (unsigned long)gridDim.x * 256ul) {
+    const unsigned long step = (unsigned long)gridDim.x * 256ul;
+    unsigned long i = blockIdx.x * 256ul + threadIdx.x;
+    for (; i + 3 * step < n; i += 4 * step) {
+        double2 x[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) x[k] = load_res(res, PREC, i + k * step);
+#pragma unroll
+        for (int k = 0; k < 4; k++) m = fmax(m, fabs(x[k].x) + fabs(x[k].y));
+    }
+    for (; i < n; i += step) {
         const double2 x = load_res(res, PREC, i);
         m = fmax(m, fabs(x.x) + fabs(x.y));
     }
+    // one atomic per work-group: on one address they take 12 ns each, and 16,384 of them (one
+    // per wave of 4,096 work-groups) took 190 us whatever the residual's size
+    __shared__ double part[4];
     for (int off = 32; off >= 1; off >>= 1) m = fmax(m, __shfl_xor(m, off));
-    if ((threadIdx.x & 63) == 0) atomicMax(out, (unsigned long long)__double_as_longlong(m));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = fmax(fmax(part[0], part[1]), fmax(part[2], part[3]));
+        atomicMax(out, (unsigned long long)__double_as_longlong(m));
+    }
 }
 
 void launch_abs_bound(hipStream_t s, int prec, unsigned long nvis, const void *res,
                       unsigned long long *out)
 {
-    const unsigned grid = (unsigned)std::min<unsigned long>(4096ul, (nvis + 255) / 256);
+    const unsigned grid = (unsigned)std::min<unsigned long>(2048ul, (nvis + 255) / 256);
     if (prec == 0)
         abs_bound_kernel<0><<<grid, 256, 0, s>>>(res, nvis, out);
     else
@@ -1208,7 +1238,7 @@ __device__ inline double wave_max(double v)
 // 38.5 (prefix products over the lanes took no longer, but round differently, and where few
 // points are sampled a last bit decides whether a variance is a number).
 // x0, x1 > 0 and the same in every lane; one wave of a work-group at a time (buf).
-__device__ inline void expint_ei_wave(double x0, double x1, double *y0, double *y1)
+__device__ __attribute__((always_inline)) inline void expint_ei_wave(double x0, double x1, double *y0, double *y1)
 {
     const double euler = 0.57721566490153286060651209008240243;
     constexpr int U = 8;
@@ -1295,7 +1325,7 @@ __device__ inline void expint_ei_wave(double x0, double x1, double *y0, double *
 // marg_position (rl2_math.h) by a wave, for an argument that is the same in all its lanes,
 // with the same bits.  The two exponential integrals of a task that ends with B <= 100 were its
 // longest serial chain, by one lane, on the critical path of the Newton pass.
-__device__ inline double marg_position_wave(double x)
+__device__ __attribute__((always_inline)) inline double marg_position_wave(double x)
 {
     const double Delta = 0.5 * 5.991;
     if (x <= Delta) return kBad;
@@ -1309,7 +1339,7 @@ __device__ inline double marg_position_wave(double x)
 // likelihood.c:174-183: L_r = log of the position-marginalised likelihood minus
 // 1/2 log det of the cross-correlation Hessian; -1e10 when the peak search failed.  Called
 // by a whole wave with the same arguments in every lane; lane 0 writes.
-__device__ inline void finish_lr(const LikLaunch &a, int item, int r, double ho,
+__device__ __attribute__((always_inline)) inline void finish_lr(const LikLaunch &a, int item, int r, double ho,
                                  double det_sigma, int iter)
 {
     double L;
@@ -3803,7 +3833,7 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_persist_kernel(Pe
 // 96 here; from 8,192 cells on (twice the cells in registers, which spill) 71, 77 and 128
 // against 75, 76 and 139, so kTaskChunks is 4.
 template <int KIND, int G, int NC>
-__global__ __launch_bounds__(kTileBS *G, NC == 1 ? 3 : 2) void lik_task_kernel(TileLaunch t)
+__global__ __launch_bounds__(kTileBS *G, NC == 1 ? 4 : 2) void lik_task_kernel(TileLaunch t)
 {
     constexpr int BS = kTileBS * G, Q = kTileMinCells / kTileBS, W = kTileBS / 64;
     constexpr int NJ = 8;
@@ -3914,6 +3944,12 @@ __global__ __launch_bounds__(kTileBS *G, NC == 1 ? 3 : 2) void lik_task_kernel(T
         const int done = pass == 0 ? newton_update<0>(S, v, &ho, &det)
                                    : newton_update<1>(S, v, &ho, &det);
         if (done) break;  // the same in every wave
+        // the state in scalar registers: the loop's vector registers hold the cells
+        S.xo = read_lane(S.xo, 0);
+        S.yo = read_lane(S.yo, 0);
+        S.norm = read_lane(S.norm, 0);
+        S.S2 = read_lane(S.S2, 0);
+        S.iter = __builtin_amdgcn_readfirstlane(S.iter);
         tab_rot_stage(R, RecCtr{rec}, gf, S.xo, S.yo, 0u, (gf + kTabRun - 1) / kTabRun - 1, false);
         __syncthreads();
         for (unsigned q = threadIdx.x; q < 2 * gf; q += BS) {

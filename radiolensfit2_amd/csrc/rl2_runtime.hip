@@ -1609,8 +1609,8 @@ int rl2_obs_add_sources(rl2_obs *obs, unsigned int ngal, const double *flux, con
                      "source upload");
     if (ok) {
         KTimer t(RL2_K_SOURCES);
-        launch_add_sources(g_stream, o.prec, o.nch, o.nrow, o.d_u, o.d_v, o.d_w, o.d_wn, o.d_spec,
-                           dg, ngal, sign, o.d_res);
+        launch_add_sources(g_stream, o.prec, o.nch, o.nrow, o.d_u, o.d_v, o.d_w, o.d_wn, o.d_invlam,
+                           o.d_spec, dg, ngal, sign, o.d_res);
     }
     ok = ok && hip_ok(hipGetLastError(), "add_sources");
     ok = hip_ok(hipStreamSynchronize(g_stream), "sync") && ok;
