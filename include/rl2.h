@@ -211,9 +211,10 @@ int rl2_synchronize(void);
  * RL2_TUNE_GRID_VARIANT: extraction gridding, runs of consecutive rows merged per thread
  *   before one LDS table update: 0 / 1 / 2 / 3 / 4 runs of 2 / 2 / 8 / 4 / 4 rows with
  *   tables of 512 / 1024 / 2048 / 1024 / 2048 slots, flushed to the facet after every
- *   channel; 5 / 6 runs of 2 / 4 rows with 1024 / 2048 slots that keep their cells across
- *   channels and are flushed only when the next channel might not fit; default 5 (the
- *   fastest with the subtraction fused into the pass).  Every
+ *   channel; 6 runs of 4 rows with 2048 slots that keep their cells across channels and are
+ *   flushed only when the next channel might not fit; 5 (default, the fastest) pairs of rows
+ *   of 1,024-row blocks with several copies of each cell's sums (plain gridding, weights and
+ *   visibilities without a finite bound: runs of 2 rows with 1024 slots, as 6).  Every
  *   variant accumulates in integers, so the facet does not depend on the order of the
  *   work-groups (variants with the same rows per work-group give the same bits).
  * RL2_TUNE_TILE_CELLS: facet cells per work-group of the tiled likelihood, a power of two

@@ -56,29 +56,46 @@ __device__ inline double rsqrt_ge1(double a)
 
 // The same model with (1 + s w |k|^2)^(-3/2) as rsqrt(den)^3 (one reciprocal square
 // root instead of a square root and a division; a few ulp from the reference's form).
-__device__ inline double model_shape_rsq(const GalaxyGeom &g, double u, double v, double wn2,
-                                         double spectra)
+// model_kk: |k|^2 of a row, the same in all its channels.
+__device__ inline double model_kk(const GalaxyGeom &g, double u, double v)
 {
     const double k1 = fma(g.e2, v, (1. + g.e1) * u);
     const double k2 = fma(1. - g.e1, v, g.e2 * u);
-    const double rr = rsqrt_ge1(fma(g.sf * wn2, fma(k1, k1, k2 * k2), 1.));
+    return fma(k1, k1, k2 * k2);
+}
+__device__ inline double model_shape_kk(const GalaxyGeom &g, double kk, double wn2, double spectra)
+{
+    const double rr = rsqrt_ge1(fma(g.sf * wn2, kk, 1.));
     return rr * rr * rr * (spectra * g.flux);
+}
+__device__ inline double model_shape_rsq(const GalaxyGeom &g, double u, double v, double wn2,
+                                         double spectra)
+{
+    return model_shape_kk(g, model_kk(g, u, v), wn2, spectra);
 }
 
 // One visibility of the post-fit update (data_processing.c:109-135): R = (R - fit) + round,
 // both models with the phase rotor of the fitted galaxy's position (p = u l + v m + w n,
 // the phase k p in revolutions is p / lambda).
+__device__ inline double2 subtract_vis_kk(const GalaxyGeom &fit, const GalaxyGeom &rnd, double p,
+                                          double kk_fit, double kk_rnd, double k2, double spectra,
+                                          double inv_lambda, double2 r)
+{
+    double sn, cs;
+    sincos_rev64(p * inv_lambda, sn, cs);
+    const double sr = model_shape_kk(rnd, kk_rnd, k2, spectra);
+    const double sfit = model_shape_kk(fit, kk_fit, k2, spectra);
+    r.x = (r.x - sfit * cs) + sr * cs;
+    r.y = (r.y - sfit * sn) + sr * sn;
+    return r;
+}
+
 __device__ inline double2 subtract_vis(const GalaxyGeom &fit, const GalaxyGeom &rnd, double p,
                                        double u, double v, double k2, double spectra,
                                        double inv_lambda, double2 r)
 {
-    double sn, cs;
-    sincos_rev64(p * inv_lambda, sn, cs);
-    const double sr = model_shape_rsq(rnd, u, v, k2, spectra);
-    const double sfit = model_shape_rsq(fit, u, v, k2, spectra);
-    r.x = (r.x - sfit * cs) + sr * cs;
-    r.y = (r.y - sfit * sn) + sr * sn;
-    return r;
+    return subtract_vis_kk(fit, rnd, p, model_kk(fit, u, v), model_kk(rnd, u, v), k2, spectra,
+                           inv_lambda, r);
 }
 
 // ------------------------------------------------------------------ sources / noise
@@ -413,9 +430,259 @@ __global__ __launch_bounds__(256) void grid_run_kernel(GridLaunch a)
     }
 }
 
+// ---- extraction's default: one LDS table per work-group with a copy of every sum per lane
+// Sorted rows put a wave's visibilities of a channel into two to four cells (64 rows of a
+// 197-dish observation into 1.7 cells at 296 columns, 3.2 at 924), so a table with one sum per
+// cell made the LDS atomics of 64 lanes wait for each other on one address: they were half of
+// the extraction.  Here lane l adds to copy l % 4 of a cell's sums, which are in different
+// banks, and the copies are added when the table is flushed.  512 threads of 2 rows and 512
+// cells of 4 copies: 60 KB, two work-groups per CU, the 16 waves that 128 registers allow.  1,024
+// rows and all channels of that array have 30 to 190 cells.  74M visibilities (complex128, 8
+// channels) take 1.09 ms (runs merged in registers, one sum per cell: 1.41; with the subtraction
+// 1.48 against 1.62), 15M in complex64 0.27 ms (0.37), 0.8M in 16 channels 31 us (51; 43
+// against 58).  What is left is FP64 arithmetic (two thirds of the issue slots) and the LDS
+// atomics.  Fewer cells (256) take 3% longer where corners of the uv plane overflow, 2 copies
+// 4%, 1 row per thread or 3 waves per SIMD 25% to 30%; loading a channel ahead gives nothing.
+// A visibility that finds no place in kCellProbes steps goes to the accumulators directly, so
+// the table has no size that must suffice, and it is flushed when three quarters are in use
+// (looked at every four channels) and at the end.  The integer sums make the facet the same
+// bit for bit however the visibilities are spread over copies and flushes.
+// Values are rounded by adding 1.5 * 2^52 (|x| 2^S < 2^51 by fx_scales, which needs finite
+// bounds: the host takes the kernel above otherwise); a NaN counts as 0, as its conversion did.
+constexpr int kCellBS = 512, kCellRows = 2, kCellSlots = 512, kCellCopies = 4, kCellProbes = 8;
+struct CellTable {
+    unsigned long long sum[3][kCellSlots * kCellCopies];  // re, im, sigma^2
+    uint32_t cnt[kCellSlots * kCellCopies];
+    uint32_t key[kCellSlots], list[kCellSlots];
+    uint32_t used;
+};
+
+__device__ inline long long fx_round51(double x, double scale)
+{
+    constexpr double kRound = 6755399441055744.;
+    return (long long)(__builtin_bit_cast(uint64_t, fma(x, scale, kRound)) -
+                       __builtin_bit_cast(uint64_t, kRound));
+}
+
+__device__ inline void cell_clear(CellTable &T)
+{
+    for (int k = threadIdx.x; k < kCellSlots * kCellCopies; k += kCellBS) {
+        T.sum[0][k] = T.sum[1][k] = T.sum[2][k] = 0ull;
+        T.cnt[k] = 0;
+    }
+    static_assert(kCellSlots <= kCellBS, "a key per thread");
+    if (threadIdx.x < kCellSlots) T.key[threadIdx.x] = kEmpty;
+    if (threadIdx.x == 0) T.used = 0;
+}
+
+__device__ inline void cell_add(CellTable &T, double *accd, unsigned long ncell, uint32_t key,
+                                long long re, long long im, long long s2, uint32_t n)
+{
+    uint32_t h = (key * 2654435761u) >> 23;
+    static_assert(kCellSlots == 1 << 9, "hash bits");
+#pragma unroll 1
+    for (int p = 0; p < kCellProbes; p++) {
+        uint32_t k = __hip_atomic_load(&T.key[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (k == kEmpty) {
+            k = atomicCAS(&T.key[h], kEmpty, key);
+            if (k == kEmpty) {
+                T.list[atomicAdd(&T.used, 1u)] = h;
+                k = key;
+            }
+        }
+        if (k == key) {
+            const uint32_t at = h * kCellCopies + (threadIdx.x & (kCellCopies - 1));
+            atomicAdd(&T.sum[0][at], (unsigned long long)re);
+            atomicAdd(&T.sum[1][at], (unsigned long long)im);
+            atomicAdd(&T.sum[2][at], (unsigned long long)s2);
+            atomicAdd(&T.cnt[at], n);
+            return;
+        }
+        h = (h + 1) & (kCellSlots - 1);
+    }
+    unsigned long long *acc = (unsigned long long *)accd;
+    fx_flush(acc + kAccReHi * ncell + key, acc + kAccReLo * ncell + key, re);
+    fx_flush(acc + kAccImHi * ncell + key, acc + kAccImLo * ncell + key, im);
+    fx_flush(acc + kAccS2Hi * ncell + key, acc + kAccS2Lo * ncell + key, s2);
+    unsafeAtomicAdd(&accd[kAccW * ncell + key], (double)n);
+}
+
+// The table's sums to the accumulators, and the table empty again; by the whole work-group,
+// with a barrier before it and the last one inside.
+__device__ inline void cell_flush(CellTable &T, double *accd, unsigned long ncell)
+{
+    const uint32_t nocc = T.used;
+    unsigned long long *acc = (unsigned long long *)accd;
+    for (uint32_t j = threadIdx.x; j < nocc * 4; j += kCellBS) {
+        const uint32_t s = T.list[j >> 2], q = j & 3, key = T.key[s];
+        unsigned long long t = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kCellCopies; i++) {  // starting at another bank for each cell
+            const uint32_t at = s * kCellCopies + ((i + s) & (kCellCopies - 1));
+            if (q < 3) {
+                t += T.sum[q][at];
+                T.sum[q][at] = 0ull;
+            } else {
+                t += T.cnt[at];
+                T.cnt[at] = 0;
+            }
+        }
+        if (q < 3)
+            fx_flush(acc + (2 * q) * ncell + key, acc + (2 * q + 1) * ncell + key, (long long)t);
+        else
+            unsafeAtomicAdd(&accd[kAccW * ncell + key], (double)t);  // integer-valued: exact
+    }
+    static_assert(kAccReHi == 0 && kAccImHi == 2 && kAccS2Hi == 4, "accumulator order");
+    __syncthreads();
+    for (uint32_t j = threadIdx.x; j < nocc; j += kCellBS) T.key[T.list[j]] = kEmpty;
+    if (threadIdx.x == 0) T.used = 0;
+    __syncthreads();
+}
+
+// One visibility of a galaxy's facet: the round model added, shifted to the galaxy
+// (source_extraction.c:51-65), as integers of the facet's scale, with its cell; false when it is
+// flagged or outside.
+struct CellTerm {
+    uint32_t key;
+    long long re, im, s2;
+};
+template <class Exact>
+__device__ inline bool cell_term(CellTerm &o, const GridLaunch &a, double u_inc, double v_inc,
+                                 double mid, double kk, double p, double2 r, float s2, double wn2,
+                                 double spectra, double inv_lambda, const Exact &exact)
+{
+    if (signbit(s2)) return false;
+    if (!cell_index_scaled(u_inc, v_inc, inv_lambda, mid, a.len, a.inc, a.facet, exact, &o.key))
+        return false;
+    const double shape = model_shape_kk(a.g, kk, wn2, spectra);
+    double sn, cs;
+    sincos_rev64(p * inv_lambda, sn, cs);  // the phase k p in revolutions is p / lambda
+    const double gre = shape * cs + r.x;
+    const double gim = shape * sn + r.y;
+    const double xr = gre * cs - gim * (-sn);
+    const double xi = gre * (-sn) + gim * cs;
+    const bool nan = __builtin_isunordered(xr, xi);
+    o.re = nan ? 0 : fx_round51(xr, a.fx_scale);
+    o.im = nan ? 0 : fx_round51(xi, a.fx_scale);
+    o.s2 = fx_round51((double)s2, a.fs_scale);  // never a NaN (pack_sigma_kernel)
+    return true;
+}
+
+// SUB: the previous galaxy's post-fit update in the same pass, as grid_run_kernel.
+template <int PREC, bool SUB>
+__global__ __launch_bounds__(kCellBS, 4) void grid_cell_kernel(GridLaunch a)
+{
+    constexpr int RPT = kCellRows;
+    static_assert(RPT == 2, "a pair of rows");
+    __shared__ CellTable T;
+    cell_clear(T);
+    // The work-groups of the sorted order's two ends first: its sparse corners, whose rows have
+    // cells of their own, take two to four times as long as the others and would otherwise run
+    // alone at the end (115 us of 270 on 29M visibilities).
+    const unsigned block =
+        blockIdx.x & 1 ? gridDim.x - 1 - blockIdx.x / 2 : blockIdx.x / 2;
+    const unsigned long row0 =
+        (unsigned long)block * (RPT * kCellBS) + (unsigned long)threadIdx.x * RPT;
+    const unsigned long ncell = (unsigned long)a.facet * a.facet;
+    const double inv_inc = 1.0 / a.inc, mid = a.len * inv_inc;
+    // What a row keeps for all channels; its u and v in metres only for the rare exact cell
+    // index, so they are read again there.  A row past the end reads the last one's values and
+    // counts as flagged.
+    double ru[RPT], rv[RPT], rp[RPT], rps[RPT], rk[RPT], rkf[RPT];
+    bool ok[RPT];
+    using Res = typename std::conditional<PREC == 0, double2, float2>::type;
+    const Res *pr[RPT];
+    const float *ps[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; k++) {
+        ok[k] = row0 + k < a.nrow;
+        const unsigned long i = ok[k] ? row0 + k : a.nrow - 1;
+        const double u = a.u[i], v = a.v[i], w = a.w[i];
+        ru[k] = u * inv_inc;
+        rv[k] = v * inv_inc;
+        rp[k] = u * a.g.l0 + v * a.g.m0 + w * a.g.n0;
+        rk[k] = model_kk(a.g, u, v);  // SUB: that of srnd too (the host checks e = 0 in both)
+        rps[k] = SUB ? u * a.sfit.l0 + v * a.sfit.m0 + w * a.sfit.n0 : 0.;
+        rkf[k] = SUB ? model_kk(a.sfit, u, v) : 0.;
+        pr[k] = (const Res *)a.res + i;
+        ps[k] = a.s2f + i;
+    }
+    __syncthreads();
+    for (unsigned c = 0; c < a.nch; c++) {
+        const double wn = a.wn[c], inv_lambda = a.inv_lambda[c];
+        const double wn2 = wn * wn, spectra = a.spec[c];
+        // both rows' values together: each line is still there for the second load
+        float vs2[RPT];
+        double2 vres[RPT];
+#pragma unroll
+        for (int k = 0; k < RPT; k++) {
+            const Res r = pr[k][(size_t)c * a.nrow];
+            const float s2 = ps[k][(size_t)c * a.nrow];
+            vres[k] = make_double2((double)r.x, (double)r.y);
+            vs2[k] = ok[k] ? s2 : -1.f;
+        }
+        if (SUB) {
+#pragma unroll
+            for (int k = 0; k < RPT; k++) {
+                const double2 r = subtract_vis_kk(a.sfit, a.srnd, rps[k], rkf[k], rk[k], wn2,
+                                                  spectra, inv_lambda, vres[k]);
+                if (ok[k]) store_res(a.res_w, PREC, (size_t)c * a.nrow + row0 + k, r);
+                // the value a separate pass would read back
+                vres[k] = PREC == 0 ? r : make_double2((double)(float)r.x, (double)(float)r.y);
+            }
+        }
+        CellTerm t[RPT];
+        bool in[RPT];
+#pragma unroll
+        for (int k = 0; k < RPT; k++) {
+            in[k] = cell_term(t[k], a, ru[k], rv[k], mid, rk[k], rp[k], vres[k], vs2[k], wn2,
+                              spectra, inv_lambda, [&](double *u, double *v) {
+                                  const unsigned long i = row0 + k;  // not flagged: a row
+                                  *u = a.u[i];
+                                  *v = a.v[i];
+                              });
+        }
+        const bool pair = in[0] && in[1] && t[0].key == t[1].key;
+        if (pair) {
+            t[0].re += t[1].re;
+            t[0].im += t[1].im;
+            t[0].s2 += t[1].s2;
+        }
+        // one call site: a lane's second visibility in another cell takes another turn
+        bool more = in[0] || in[1];
+        bool first = in[0];
+        while (more) {
+            const uint32_t key = first ? t[0].key : t[1].key;
+            const long long re = first ? t[0].re : t[1].re, im = first ? t[0].im : t[1].im,
+                            s2 = first ? t[0].s2 : t[1].s2;
+            cell_add(T, a.acc, ncell, key, re, im, s2, first && pair ? 2u : 1u);
+            more = first && in[1] && !pair;
+            first = false;
+        }
+        if ((c & 3) == 3 && c + 1 < a.nch) {
+            __syncthreads();
+            const uint32_t used = T.used;
+            __syncthreads();  // every thread has read it before any adds a cell
+            if (used > kCellSlots * 3 / 4) cell_flush(T, a.acc, ncell);
+        }
+    }
+    __syncthreads();
+    cell_flush(T, a.acc, ncell);
+}
+
 template <int MODE, int PREC>
 static void launch_grid_variant(hipStream_t s, const GridLaunch &a)
 {
+    if (MODE == 0 && tuning().grid_variant == 5 && a.finite &&
+        !(a.sub && (a.g.e1 != 0. || a.g.e2 != 0. || a.srnd.e1 != 0. || a.srnd.e2 != 0.))) {
+        constexpr unsigned rows = kCellRows * kCellBS;
+        const dim3 grid((unsigned)((a.nrow + rows - 1) / rows));
+        if (a.sub)
+            grid_cell_kernel<PREC, true><<<grid, kCellBS, 0, s>>>(a);
+        else
+            grid_cell_kernel<PREC, false><<<grid, kCellBS, 0, s>>>(a);
+        return;
+    }
     if (tuning().grid_variant == 5) {
         // runs of 2 rows, 1024 slots, flushed when another channel might not fit
         constexpr int RPT = 2;
@@ -4574,6 +4841,7 @@ __global__ void pack_sigma_kernel(unsigned nch, unsigned long nrow, const uint32
     for (unsigned c = 0; c < nch; c++) {
         float sg = sigma2[(size_t)c * nrow + src];
         bool fl = flag && flag[(size_t)c * nrow + src];
+        if (isnan(sg) && !signbit(sg)) sg = 0.f;  // adds nothing, as its conversion did
         s2f[(size_t)c * nrow + i] = fl ? -fabsf(sg) - 0.0f : sg;
     }
 }

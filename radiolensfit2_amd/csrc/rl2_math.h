@@ -115,25 +115,40 @@ RL2_HD void sincos_rev64(double t, double &sn, double &cs)
     cs = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, b) ^ (((k + 1) & 2) << 62));
 }
 
-// cell_index (evaluate_uv_grid.c:166-178) with the two divisions by the cell size replaced
-// by products with its reciprocal.  The product is within a few ulp of the correctly
-// rounded quotient, so their integer parts can only differ when the quotient lies within
-// that distance of an integer; there (|q - rint(q)| < 1e-9, far above the few-ulp error
-// for quotients below 2^21) the exact division is taken, so the cell is always the
-// reference's.
-RL2_HD bool cell_index_fast(double u, double v, double inv_lambda, double len, double inc,
-                            double inv_inc, unsigned int facet, uint32_t *pc_out)
+// cell_index (evaluate_uv_grid.c:166-178) with each quotient (u / lambda + len) / inc as one
+// fused product, (u / inc) / lambda + len / inc, whose factors do not depend on the channel.
+// It is within a few ulp of the correctly rounded quotient, so their integer parts can only
+// differ when it lies within that distance of an integer; there (|q - rint(q)| < 1e-9, far
+// above the error for quotients below 2^20) the reference's sum and division are taken, so the
+// cell is always the reference's.
+// exact(&u, &v): the row's coordinates in metres, for the division.
+template <class Exact>
+RL2_HD bool cell_index_scaled(double u_inc, double v_inc, double inv_lambda, double mid, double len,
+                              double inc, unsigned int facet, const Exact &exact,
+                              uint32_t *pc_out)
 {
-    const double a = u * inv_lambda + len;
-    const double b = v * inv_lambda + len;
-    double qa = a * inv_inc, qb = b * inv_inc;
-    if (fabs(qa - rint(qa)) < 1e-9) qa = a / inc;
-    if (fabs(qb - rint(qb)) < 1e-9) qb = b / inc;
+    double qa = fma(u_inc, inv_lambda, mid), qb = fma(v_inc, inv_lambda, mid);
+    if (fabs(qa - rint(qa)) < 1e-9 || fabs(qb - rint(qb)) < 1e-9) {
+        double u, v;
+        exact(&u, &v);
+        qa = (u * inv_lambda + len) / inc;
+        qb = (v * inv_lambda + len) / inc;
+    }
     const unsigned int pu = (unsigned int)qa;
     const unsigned int pv = (unsigned int)qb;
     const unsigned long long pc = (unsigned long long)pv * facet + pu;
     *pc_out = (uint32_t)pc;
     return pc < (unsigned long long)facet * facet;
+}
+RL2_HD bool cell_index_fast(double u, double v, double inv_lambda, double len, double inc,
+                            double inv_inc, unsigned int facet, uint32_t *pc_out)
+{
+    return cell_index_scaled(u * inv_inc, v * inv_inc, inv_lambda, len * inv_inc, len, inc, facet,
+                             [&](double *pu, double *pv) {
+                                 *pu = u;
+                                 *pv = v;
+                             },
+                             pc_out);
 }
 
 // Philox4x32-10 counter-based generator (Salmon, Moraes, Dror and Shaw, SC'11): ten rounds of

@@ -499,7 +499,9 @@ bool obs_extract(Obs &o, int slot, double l0, double m0, double flux, double R_m
     a.acc = s.acc;
     // a visibility that is gridded is at most |round model| + |residual| per component
     if (sub) o.res_bound += 3. * fabs(sub->flux) * o.spec_max;
-    const AccScale sc = fx_scales(fabs(flux) * o.spec_max + o.res_bound, o.s2_max, -1, o.nch);
+    const double bound = fabs(flux) * o.spec_max + o.res_bound;
+    const AccScale sc = fx_scales(bound, o.s2_max, -1, o.nch);
+    a.finite = std::isfinite(bound) && std::isfinite(o.s2_max);
     a.fx_scale = sc.fx_scale;
     a.fs_scale = sc.fs_scale;
     if (sub) {  // the previous galaxy's post-fit update in the same pass
