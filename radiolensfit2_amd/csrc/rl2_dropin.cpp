@@ -350,8 +350,15 @@ static unsigned grid_natural(int mode, const double *wavenumbers, unsigned nch, 
     a.fx_scale = sc.fx_scale;
     a.fs_scale = sc.fs_scale;
     launch_grid(stream(), a);
-    launch_compact(stream(), acc.p, sizeg, len, cu.p, cv.p, cre.p, cim.p, cs2.p, nullptr, nullptr,
-                   dn.p, csw.p, scan.p, &sc);
+    CompactOut out = {};
+    out.uu = cu.p;
+    out.vv = cv.p;
+    out.dre = cre.p;
+    out.dim = cim.p;
+    out.s2 = cs2.p;
+    out.n_out = dn.p;
+    out.sum_w = csw.p;
+    launch_compact(stream(), acc.p, sizeg, len, out, scan.p, &sc);
     unsigned n = 0;
     if (!dn.down(&n, 1) || !sync_ok()) {
         report("gridding");
@@ -411,8 +418,14 @@ static unsigned compact_host(unsigned sizeg, double len, const double *re, const
     DBuf<unsigned> scan(compact_scratch_words(sizeg) + 1), dn(1);
     if (!allocated(dacc, cu, cv, cre, cim, cs2, scan, dn) || !dacc.up(acc.data(), 4 * ncell))
         return 0;
-    launch_compact(stream(), dacc.p, sizeg, len, cu.p, cv.p, cre.p, cim.p, cs2.p, nullptr, nullptr,
-                   dn.p, nullptr, scan.p, nullptr);
+    CompactOut out = {};
+    out.uu = cu.p;
+    out.vv = cv.p;
+    out.dre = cre.p;
+    out.dim = cim.p;
+    out.s2 = cs2.p;
+    out.n_out = dn.p;
+    launch_compact(stream(), dacc.p, sizeg, len, out, scan.p, nullptr);
     unsigned n = 0;
     if (!dn.down(&n, 1) || !sync_ok()) return 0;
     std::vector<double> vr(n), vi(n);
@@ -478,7 +491,8 @@ void source_extraction(int, unsigned int facet, likelihood_params *par, complexd
         return;
     }
     if (rl2_obs_set_vis(g_obs.get(), (const double *)visData, (const double *)visSkyMod) != RL2_OK ||
-        !o->ensure_slots(1) || !obs_extract(*o, 0, l0, m0, flux, mu, facet, true, e1, e2)) {
+        !o->ensure_slots(1) || !obs_extract(*o, 0, l0, m0, flux, mu, facet,
+                                            ExtractCopy::weights, e1, e2)) {
         report("source_extraction");
         return;
     }

@@ -35,9 +35,26 @@ struct FacetDev {
     const uint32_t *loff;
     unsigned int grid_facet;
     unsigned int pad0;
-    unsigned int n;
-    unsigned int pad;
     double rprior[kMaxR];      // log prior per scalelength index
+    unsigned int n;            // last: written on the device, the rest pushed by the host
+    unsigned int pad;
+};
+
+// Where a compaction writes a facet's n cells, in row-major order.
+struct CompactOut {
+    double *uu, *vv, *dre, *dim, *s2;
+    unsigned *n_out;                   // the cell count
+    uint32_t *cid = nullptr;           // grid structure (FacetDev), or null
+    double *ctr = nullptr;
+    float4 *pk = nullptr;              // with invs2, invs2_64, dc, loff: FacetDev's copies
+    float *invs2 = nullptr;
+    double *invs2_64 = nullptr;
+    double2 *dc = nullptr;
+    uint32_t *loff = nullptr;
+    double *sum_w = nullptr;           // dense weights (facet^2)
+    unsigned *n_host = nullptr;        // the count again, in pinned host memory
+    double2 *h_vis = nullptr;          // with h_s2, h_uu, h_vv: the cells, in pinned host memory
+    double *h_s2 = nullptr, *h_uu = nullptr, *h_vv = nullptr;
 };
 
 // One likelihood evaluation request.
@@ -170,16 +187,8 @@ struct BatchSub {
 struct BatchCompact {
     double *acc;
     double fx_unscale, fs_unscale;
-    double *uu, *vv, *dre, *dim, *s2;
-    uint32_t *cid;
-    double *ctr;
-    double2 *dc;
-    uint32_t *loff;
-    float4 *pk;
-    float *invs2;
-    double *invs2_64;
-    unsigned *n_out;            // the slot descriptor's cell count
-    unsigned *scan;             // block counts, compact_scratch_words(facet) words
+    CompactOut out;
+    unsigned *scan;             // tile counts, compact_scratch_words(facet) words
     unsigned facet;
     unsigned pad;
 };
@@ -205,7 +214,7 @@ struct GridBatchLaunch {
                                 // launch, and the launch leaves them zero again
     unsigned ntiles;
 };
-// The batch's compactions and FP32 copies: four launches over ncap targets of facets up to
+// The batch's compactions and FP32 copies: two launches over ncap targets of facets up to
 // fmax (targets beyond desc->ntarget and blocks beyond a facet exit at once).
 void launch_compact_batch(hipStream_t s, const BatchDesc *desc, unsigned ncap, unsigned fmax,
                           double len);
@@ -248,20 +257,13 @@ Tuning &tuning();
 // Compaction of dense accumulators into the facet arrays; clears the accumulators.
 // fx: the integer accumulators of launch_grid with these scales; null: four double arrays
 // acc[4][facet^2] (re, im, sigma^2, weight) given by a caller.
-// n_out (device) receives the number of non-empty cells. sum_w_dense (optional, device)
-// receives the dense weights before clearing.
-// cid / ctr (optional): packed row and column of each compacted cell, and the centre
-// coordinate of every grid index (facet entries).
-void launch_compact(hipStream_t s, double *acc, unsigned facet, double len, double *uu,
-                    double *vv, double *dre, double *dim, double *s2, uint32_t *cid, double *ctr,
-                    unsigned *n_out,
-                    double *sum_w_dense, unsigned *scratch_blocks, const AccScale *fx);
+void launch_compact(hipStream_t s, double *acc, unsigned facet, double len, const CompactOut &out,
+                    unsigned *scratch, const AccScale *fx);
 size_t compact_scratch_words(unsigned facet);
-// FP32 packing of a compacted facet (count read from the device descriptor).
-void launch_pack_facet(hipStream_t s, const FacetDev *dfacet, unsigned cap, const double *uu,
-                       const double *vv, const double *dre, const double *dim, const double *s2,
-                       float4 *pk, float *invs2, double *invs2_64, const uint32_t *cid,
-                       unsigned facet, double2 *dc, uint32_t *loff);
+// FP32 and packed copies of a facet of n cells without grid structure.
+void launch_pack_facet(hipStream_t s, unsigned n, const double *uu, const double *vv,
+                       const double *dre, const double *dim, const double *s2, float4 *pk,
+                       float *invs2, double *invs2_64, double2 *dc);
 
 struct TileTask {
     double xo, yo;             // position offset of the current Newton iterate

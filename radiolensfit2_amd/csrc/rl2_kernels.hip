@@ -743,63 +743,51 @@ void launch_grid(hipStream_t s, const GridLaunch &a)
 // ------------------------------------------------------------------ compaction
 // Cells with weight != 0 in row-major order (evaluate_uv_grid.c:196-210 and :113-133):
 //   vis = sum_vis * w / sum_sigma2, sigma2 = sum_sigma2 / w^2, (u,v) = cell centre.
-constexpr int kCompactBS = 256, kCompactPT = 16, kCompactTile = kCompactBS * kCompactPT;
+// Two launches: the cells of every tile are counted, then a work-group per tile adds the counts
+// of the tiles before it (at most a few hundred words from L2, instead of a scan of its own)
+// and writes its cells with every copy of them that the likelihood reads.  Bound by the latency
+// of its loads: consecutive lanes take consecutive cells, kCompactPT loads in flight each.
+// An extracted facet of 1,024 grid cells takes 4 + 6 us (a count, a scan, a write of 16 cells
+// in a row per thread and a copying launch: 5 + 4 + 20 + 5 us), of 60,000 cells 5 + 13 (6 + 5 +
+// 61 + 6).
+constexpr int kCompactBS = 256, kCompactPT = 4, kCompactTile = kCompactBS * kCompactPT;
+constexpr int kCompactW = kCompactBS / 64;
+
+__host__ __device__ inline unsigned compact_tiles(unsigned long ncell)
+{
+    return (unsigned)((ncell + kCompactTile - 1) / kCompactTile);
+}
 
 size_t compact_scratch_words(unsigned facet)
 {
-    size_t ncell = (size_t)facet * facet;
-    return (ncell + kCompactTile - 1) / kCompactTile + 1;
+    return compact_tiles((unsigned long)facet * facet) + 1;
+}
+
+__device__ inline void compact_count_tile(unsigned blk, const double *acc_w, unsigned long ncell,
+                                          unsigned *bcount)
+{
+    __shared__ unsigned part[kCompactW];
+    const unsigned long base = (unsigned long)blk * kCompactTile + threadIdx.x;
+    unsigned cnt = 0;
+#pragma unroll
+    for (int k = 0; k < kCompactPT; k++) {
+        const unsigned long p = base + k * kCompactBS;
+        cnt += (unsigned)__popcll(__ballot(p < ncell && acc_w[p < ncell ? p : 0] != 0.));
+    }
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = cnt;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned t = 0;
+        for (int i = 0; i < kCompactW; i++) t += part[i];
+        bcount[blk] = t;
+    }
 }
 
 __global__ __launch_bounds__(kCompactBS) void compact_count_kernel(const double *acc_w,
                                                                    unsigned long ncell,
                                                                    unsigned *bcount)
 {
-    __shared__ unsigned part[kCompactBS / 64];
-    unsigned long base = (unsigned long)blockIdx.x * kCompactTile + threadIdx.x * kCompactPT;
-    unsigned cnt = 0;
-    for (int k = 0; k < kCompactPT; k++) {
-        unsigned long p = base + k;
-        if (p < ncell && acc_w[p] != 0.) cnt++;
-    }
-    for (int off = 32; off >= 1; off >>= 1) cnt += __shfl_xor(cnt, off);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = cnt;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned t = 0;
-        for (int i = 0; i < kCompactBS / 64; i++) t += part[i];
-        bcount[blockIdx.x] = t;
-    }
-}
-
-// exclusive scan of nb block counts in place (single work-group), total -> bcount[nb]
-__global__ __launch_bounds__(1024) void compact_scan_kernel(unsigned *bcount, unsigned nb,
-                                                            unsigned *n_out)
-{
-    __shared__ unsigned buf[1024];
-    __shared__ unsigned carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (unsigned base = 0; base < nb; base += 1024) {
-        unsigned i = base + threadIdx.x;
-        unsigned x = (i < nb) ? bcount[i] : 0;
-        buf[threadIdx.x] = x;
-        __syncthreads();
-        for (unsigned off = 1; off < 1024; off <<= 1) {
-            unsigned t = (threadIdx.x >= off) ? buf[threadIdx.x - off] : 0;
-            __syncthreads();
-            buf[threadIdx.x] += t;
-            __syncthreads();
-        }
-        if (i < nb) bcount[i] = carry + buf[threadIdx.x] - x;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry += buf[1023];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        bcount[nb] = carry;
-        *n_out = carry;
-    }
+    compact_count_tile(blockIdx.x, acc_w, ncell, bcount);
 }
 
 // Accumulators of cell p: FX (device gridding) the integer layout above, scaled back by
@@ -838,87 +826,119 @@ __device__ inline void acc_clear(double *acc, unsigned long ncell, unsigned long
     }
 }
 
-// One work-group's tile of the compaction (block `blk` of the nb blocks of one facet).
-template <bool FX>
-__device__ inline void compact_write_tile(
-    unsigned blk, unsigned nb, double *acc, unsigned facet, unsigned long ncell, double len,
-    const unsigned *boff, double *uu, double *vv, double *dre, double *dim, double *s2o,
-    uint32_t *cid, double *ctr, double *sum_w_dense, double fx_unscale, double fs_unscale,
-    unsigned *tscan)
+// Cell i's packed data and record offsets for the fused Newton passes (cell n: the zero pad
+// cell); offsets only for grid facets with records (facet <= kRecFacet).
+__device__ inline void pack_cell_records(unsigned i, double re, double im, const uint32_t *cid,
+                                         uint32_t c, unsigned facet, double2 *dc, uint32_t *loff)
 {
+    dc[i] = make_double2(re, im);
+    if (cid && facet <= kRecFacet)
+        loff[i] = ((c >> 16) * kRecBytes) << 16 | (c & 0xffffu) * kRecBytes;
+}
+
+// One work-group's tile of the compaction (tile `blk` of the nb tiles of one facet).
+template <bool FX>
+__device__ inline void compact_write_tile(unsigned blk, unsigned nb, double *acc, unsigned facet,
+                                          unsigned long ncell, double len, const unsigned *bcount,
+                                          const CompactOut &C, double fx_unscale,
+                                          double fs_unscale)
+{
+    __shared__ unsigned part[kCompactW], count[kCompactPT][kCompactW];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const double *acc_w = acc + (FX ? kAccW : 3) * ncell;
-    unsigned long base = (unsigned long)blk * kCompactTile + threadIdx.x * kCompactPT;
-    unsigned cnt = 0;
+    const unsigned long base = (unsigned long)blk * kCompactTile + threadIdx.x;
+    double wgt[kCompactPT];
+#pragma unroll
     for (int k = 0; k < kCompactPT; k++) {
-        unsigned long p = base + k;
-        if (p < ncell && acc_w[p] != 0.) cnt++;
+        const unsigned long p = base + k * kCompactBS;
+        wgt[k] = p < ncell ? acc_w[p] : 0.;
     }
-    tscan[threadIdx.x] = cnt;
+    unsigned before = 0;
+    for (unsigned t = threadIdx.x; t < blk; t += kCompactBS) before += bcount[t];
+    for (int off = 32; off >= 1; off >>= 1) before += __shfl_xor(before, off);
+    if (lane == 0) part[wave] = before;
+    unsigned rank[kCompactPT];
+#pragma unroll
+    for (int k = 0; k < kCompactPT; k++) {
+        const unsigned long long mask = __ballot(wgt[k] != 0.);
+        rank[k] = (unsigned)__popcll(mask & ((1ull << lane) - 1ull));
+        if (lane == 0) count[k][wave] = (unsigned)__popcll(mask);
+    }
     __syncthreads();
-    for (int off = 1; off < kCompactBS; off <<= 1) {
-        unsigned t = (threadIdx.x >= (unsigned)off) ? tscan[threadIdx.x - off] : 0;
-        __syncthreads();
-        tscan[threadIdx.x] += t;
-        __syncthreads();
-    }
-    unsigned n = boff[blk] + tscan[threadIdx.x] - cnt;
+    unsigned n = 0;
+#pragma unroll
+    for (int w = 0; w < kCompactW; w++) n += part[w];
     const double inc = 2 * len / facet;
-    if (cid && blk == 0 && threadIdx.x == 0) {
+    if (C.ctr) {  // centre of grid index k, the same expression as uu / vv below
+        const unsigned k = blk * kCompactBS + threadIdx.x;
+        if (k < facet) C.ctr[k] = (k + 0.5) * inc - len;
+    }
+#pragma unroll
+    for (int k = 0; k < kCompactPT; k++) {
+        const unsigned long p = base + k * kCompactBS;
+        unsigned at = n + rank[k];
+#pragma unroll
+        for (int w = 0; w < kCompactW; w++) {
+            const unsigned c = count[k][w];
+            at += w < wave ? c : 0;
+            n += c;
+        }
+        if (C.sum_w && p < ncell) C.sum_w[p] = wgt[k];
+        if (wgt[k] == 0.) continue;
+        double re, im, sg;
+        acc_read<FX>(acc, ncell, p, fx_unscale, fs_unscale, re, im, sg);
+        const double dre = re * wgt[k] / sg, dim = im * wgt[k] / sg;
+        const double s2 = sg / (wgt[k] * wgt[k]);
+        const unsigned q = (unsigned)p, j = q / facet, i = q - j * facet;
+        const double u = (i + 0.5) * inc - len, v = (j + 0.5) * inc - len;
+        const uint32_t id = (j << 16) | i;
+        C.dre[at] = dre;
+        C.dim[at] = dim;
+        C.s2[at] = s2;
+        C.uu[at] = u;
+        C.vv[at] = v;
+        if (C.cid) C.cid[at] = id;
+        if (C.pk) {
+            const double w = 1.0 / s2;
+            C.pk[at] = make_float4((float)u, (float)v, (float)dre, (float)dim);
+            C.invs2[at] = (float)w;
+            C.invs2_64[at] = w;
+            pack_cell_records(at, dre, dim, C.cid, id, facet, C.dc, C.loff);
+        }
+        if (C.h_vis) {
+            C.h_vis[at] = make_double2(dre, dim);
+            C.h_s2[at] = s2;
+            C.h_uu[at] = u;
+            C.h_vv[at] = v;
+        }
+        acc_clear<FX>(acc, ncell, p);
+    }
+    if (blk == nb - 1 && threadIdx.x == 0) {
+        *C.n_out = n;
+        if (C.n_host) *C.n_host = n;
         // zero pad cell after the last one (the arrays hold facet^2 + 1 entries): lanes past
         // the end of a chunk read it instead of masking their data
-        const unsigned nt = boff[nb];
-        dre[nt] = 0.;
-        dim[nt] = 0.;
-        cid[nt] = 0;
-    }
-    if (ctr) {  // centre of grid index k, the same expression as uu / vv below
-        const unsigned k = blk * kCompactBS + threadIdx.x;
-        if (k < facet) ctr[k] = (k + 0.5) * inc - len;
-    }
-    for (int k = 0; k < kCompactPT; k++) {
-        unsigned long p = base + k;
-        if (p >= ncell) break;
-        double wgt = acc_w[p];
-        if (sum_w_dense) sum_w_dense[p] = wgt;
-        if (wgt != 0.) {
-            double re, im, sg;
-            acc_read<FX>(acc, ncell, p, fx_unscale, fs_unscale, re, im, sg);
-            dre[n] = re * wgt / sg;
-            dim[n] = im * wgt / sg;
-            s2o[n] = sg / (wgt * wgt);
-            unsigned j = (unsigned)(p / facet), i = (unsigned)(p % facet);
-            uu[n] = (i + 0.5) * inc - len;
-            vv[n] = (j + 0.5) * inc - len;
-            if (cid) cid[n] = (j << 16) | i;
-            n++;
-            acc_clear<FX>(acc, ncell, p);
+        if (C.cid) {
+            C.dre[n] = 0.;
+            C.dim[n] = 0.;
+            C.cid[n] = 0;
+        }
+        if (C.pk) {
+            C.invs2_64[n] = 0.;
+            pack_cell_records(n, 0., 0., C.cid, 0u, facet, C.dc, C.loff);
         }
     }
 }
 
 template <bool FX>
-__global__ __launch_bounds__(kCompactBS) void compact_write_kernel(
-    double *acc, unsigned facet, unsigned long ncell, double len, const unsigned *boff,
-    double *uu, double *vv, double *dre, double *dim, double *s2o, uint32_t *cid, double *ctr,
-    double *sum_w_dense, double fx_unscale, double fs_unscale)
+__global__ __launch_bounds__(kCompactBS) void compact_write_kernel(double *acc, unsigned facet,
+                                                                   unsigned long ncell, double len,
+                                                                   const unsigned *bcount,
+                                                                   CompactOut C, double fx_unscale,
+                                                                   double fs_unscale)
 {
-    __shared__ unsigned tscan[kCompactBS];
-    compact_write_tile<FX>(blockIdx.x, gridDim.x, acc, facet, ncell, len, boff, uu, vv, dre, dim,
-                           s2o, cid, ctr, sum_w_dense, fx_unscale, fs_unscale, tscan);
-}
-
-// The packed data and record offsets of the fused Newton passes (cell i and the zero pad
-// cell n); offsets only for grid facets with records (facet <= kRecFacet).
-__device__ inline void pack_cell_records(unsigned i, unsigned n, const double *dre,
-                                         const double *dim, const uint32_t *cid, unsigned facet,
-                                         double2 *dc, uint32_t *loff)
-{
-    const bool in = i < n;
-    dc[i] = in ? make_double2(dre[i], dim[i]) : make_double2(0., 0.);
-    if (cid && facet <= kRecFacet) {
-        const uint32_t c = in ? cid[i] : 0u;
-        loff[i] = ((c >> 16) * kRecBytes) << 16 | (c & 0xffffu) * kRecBytes;
-    }
+    compact_write_tile<FX>(blockIdx.x, gridDim.x, acc, facet, ncell, len, bcount, C, fx_unscale,
+                           fs_unscale);
 }
 
 // ---- batched compaction: grid.y = target of a BatchDesc; targets beyond desc->ntarget and
@@ -929,58 +949,8 @@ __global__ __launch_bounds__(kCompactBS) void compact_count_batch_kernel(const B
     if (t >= desc->ntarget) return;
     const BatchCompact &C = desc->compact[t];
     const unsigned long ncell = (unsigned long)C.facet * C.facet;
-    const unsigned nb = (unsigned)((ncell + kCompactTile - 1) / kCompactTile);
-    if (blockIdx.x >= nb) return;
-    __shared__ unsigned part[kCompactBS / 64];
-    const double *acc_w = C.acc + kAccW * ncell;
-    unsigned long base = (unsigned long)blockIdx.x * kCompactTile + threadIdx.x * kCompactPT;
-    unsigned cnt = 0;
-    for (int k = 0; k < kCompactPT; k++) {
-        unsigned long p = base + k;
-        if (p < ncell && acc_w[p] != 0.) cnt++;
-    }
-    for (int off = 32; off >= 1; off >>= 1) cnt += __shfl_xor(cnt, off);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = cnt;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned tt = 0;
-        for (int i = 0; i < kCompactBS / 64; i++) tt += part[i];
-        C.scan[blockIdx.x] = tt;
-    }
-}
-
-__global__ __launch_bounds__(1024) void compact_scan_batch_kernel(const BatchDesc *desc)
-{
-    const unsigned t = blockIdx.x;
-    if (t >= desc->ntarget) return;
-    const BatchCompact &C = desc->compact[t];
-    const unsigned long ncell = (unsigned long)C.facet * C.facet;
-    const unsigned nb = (unsigned)((ncell + kCompactTile - 1) / kCompactTile);
-    unsigned *bcount = C.scan;
-    __shared__ unsigned buf[1024];
-    __shared__ unsigned carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (unsigned base = 0; base < nb; base += 1024) {
-        unsigned i = base + threadIdx.x;
-        unsigned x = (i < nb) ? bcount[i] : 0;
-        buf[threadIdx.x] = x;
-        __syncthreads();
-        for (unsigned off = 1; off < 1024; off <<= 1) {
-            unsigned tt = (threadIdx.x >= off) ? buf[threadIdx.x - off] : 0;
-            __syncthreads();
-            buf[threadIdx.x] += tt;
-            __syncthreads();
-        }
-        if (i < nb) bcount[i] = carry + buf[threadIdx.x] - x;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry += buf[1023];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        bcount[nb] = carry;
-        *C.n_out = carry;
-    }
+    if (blockIdx.x >= compact_tiles(ncell)) return;
+    compact_count_tile(blockIdx.x, C.acc + kAccW * ncell, ncell, C.scan);
 }
 
 __global__ __launch_bounds__(kCompactBS) void compact_write_batch_kernel(const BatchDesc *desc,
@@ -990,43 +960,19 @@ __global__ __launch_bounds__(kCompactBS) void compact_write_batch_kernel(const B
     if (t >= desc->ntarget) return;
     const BatchCompact &C = desc->compact[t];
     const unsigned long ncell = (unsigned long)C.facet * C.facet;
-    const unsigned nb = (unsigned)((ncell + kCompactTile - 1) / kCompactTile);
+    const unsigned nb = compact_tiles(ncell);
     if (blockIdx.x >= nb) return;
-    __shared__ unsigned tscan[kCompactBS];
-    compact_write_tile<true>(blockIdx.x, nb, C.acc, C.facet, ncell, len, C.scan, C.uu, C.vv,
-                             C.dre, C.dim, C.s2, C.cid, C.ctr, nullptr, C.fx_unscale,
-                             C.fs_unscale, tscan);
-}
-
-__global__ void pack_facet_batch_kernel(const BatchDesc *desc)
-{
-    const unsigned t = blockIdx.y;
-    if (t >= desc->ntarget) return;
-    const BatchCompact &C = desc->compact[t];
-    const unsigned n = *C.n_out;
-    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        C.pk[i] = make_float4((float)C.uu[i], (float)C.vv[i], (float)C.dre[i], (float)C.dim[i]);
-        const double w = 1.0 / C.s2[i];
-        C.invs2[i] = (float)w;
-        C.invs2_64[i] = w;
-        pack_cell_records(i, n, C.dre, C.dim, C.cid, C.facet, C.dc, C.loff);
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {  // the zero pad cell
-        C.invs2_64[n] = 0.;
-        pack_cell_records(n, n, C.dre, C.dim, C.cid, C.facet, C.dc, C.loff);
-    }
+    const CompactOut out = C.out;  // in registers: its stores must not reload the descriptor
+    compact_write_tile<true>(blockIdx.x, nb, C.acc, C.facet, ncell, len, C.scan, out,
+                             C.fx_unscale, C.fs_unscale);
 }
 
 void launch_compact_batch(hipStream_t s, const BatchDesc *desc, unsigned ncap, unsigned fmax,
                           double len)
 {
-    const unsigned long ncell = (unsigned long)fmax * fmax;
-    const unsigned nb = (unsigned)((ncell + kCompactTile - 1) / kCompactTile);
+    const unsigned nb = compact_tiles((unsigned long)fmax * fmax);
     compact_count_batch_kernel<<<dim3(nb, ncap), kCompactBS, 0, s>>>(desc);
-    compact_scan_batch_kernel<<<ncap, 1024, 0, s>>>(desc);
     compact_write_batch_kernel<<<dim3(nb, ncap), kCompactBS, 0, s>>>(desc, len);
-    const unsigned pb = std::min(256u, (unsigned)((ncell + 255) / 256) + 1);
-    pack_facet_batch_kernel<<<dim3(pb, ncap), 256, 0, s>>>(desc);
 }
 
 size_t grid_acc_words(unsigned facet) { return (size_t)kAccWords * facet * facet; }
@@ -1323,24 +1269,20 @@ void launch_abs_bound(hipStream_t s, int prec, unsigned long nvis, const void *r
         abs_bound_kernel<1><<<grid, 256, 0, s>>>(res, nvis, out);
 }
 
-void launch_compact(hipStream_t s, double *acc, unsigned facet, double len, double *uu,
-                    double *vv, double *dre, double *dim, double *s2, uint32_t *cid, double *ctr,
-                    unsigned *n_out, double *sum_w_dense, unsigned *scratch, const AccScale *fx)
+void launch_compact(hipStream_t s, double *acc, unsigned facet, double len, const CompactOut &out,
+                    unsigned *scratch, const AccScale *fx)
 {
-    unsigned long ncell = (unsigned long)facet * facet;
-    unsigned nb = (unsigned)((ncell + kCompactTile - 1) / kCompactTile);
-    // ctr needs a thread per grid index: nb * kCompactBS = ceil(facet^2 / 4096) * 256 >= facet
+    const unsigned long ncell = (unsigned long)facet * facet;
+    const unsigned nb = compact_tiles(ncell);
+    // ctr needs a thread per grid index: nb * kCompactBS = ceil(facet^2 / 1024) * 256 >= facet
     // for every facet size
     compact_count_kernel<<<nb, kCompactBS, 0, s>>>(acc + (fx ? kAccW : 3) * ncell, ncell, scratch);
-    compact_scan_kernel<<<1, 1024, 0, s>>>(scratch, nb, n_out);
     if (fx)
         compact_write_kernel<true><<<nb, kCompactBS, 0, s>>>(
-            acc, facet, ncell, len, scratch, uu, vv, dre, dim, s2, cid, ctr, sum_w_dense,
-            1.0 / fx->fx_scale, 1.0 / fx->fs_scale);
+            acc, facet, ncell, len, scratch, out, 1.0 / fx->fx_scale, 1.0 / fx->fs_scale);
     else
-        compact_write_kernel<false><<<nb, kCompactBS, 0, s>>>(
-            acc, facet, ncell, len, scratch, uu, vv, dre, dim, s2, cid, ctr, sum_w_dense, 1.0,
-            1.0);
+        compact_write_kernel<false><<<nb, kCompactBS, 0, s>>>(acc, facet, ncell, len, scratch, out,
+                                                              1.0, 1.0);
 }
 
 // ------------------------------------------------------------------ likelihood (K3)
@@ -1932,34 +1874,30 @@ void launch_likelihood(hipStream_t s, const LikLaunch &a)
     }
 }
 
-__global__ void pack_facet_kernel(const FacetDev *dfacet, const double *uu, const double *vv,
+// The FP32 and packed copies of a facet given by a caller (compaction writes an extracted one's).
+__global__ void pack_facet_kernel(unsigned n, const double *uu, const double *vv,
                                   const double *dre, const double *dim, const double *s2,
-                                  float4 *pk, float *invs2, double *invs2_64,
-                                  const uint32_t *cid, unsigned facet, double2 *dc,
-                                  uint32_t *loff)
+                                  float4 *pk, float *invs2, double *invs2_64, double2 *dc)
 {
-    const unsigned n = dfacet->n;
     for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         pk[i] = make_float4((float)uu[i], (float)vv[i], (float)dre[i], (float)dim[i]);
         const double w = 1.0 / s2[i];
         invs2[i] = (float)w;
         invs2_64[i] = w;
-        pack_cell_records(i, n, dre, dim, cid, facet, dc, loff);
+        pack_cell_records(i, dre[i], dim[i], nullptr, 0u, 0u, dc, nullptr);
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {  // the zero pad cell
         invs2_64[n] = 0.;
-        pack_cell_records(n, n, dre, dim, cid, facet, dc, loff);
+        pack_cell_records(n, 0., 0., nullptr, 0u, 0u, dc, nullptr);
     }
 }
 
-void launch_pack_facet(hipStream_t s, const FacetDev *dfacet, unsigned cap, const double *uu,
-                       const double *vv, const double *dre, const double *dim, const double *s2,
-                       float4 *pk, float *invs2, double *invs2_64, const uint32_t *cid,
-                       unsigned facet, double2 *dc, uint32_t *loff)
+void launch_pack_facet(hipStream_t s, unsigned n, const double *uu, const double *vv,
+                       const double *dre, const double *dim, const double *s2, float4 *pk,
+                       float *invs2, double *invs2_64, double2 *dc)
 {
-    unsigned blocks = std::min(2048u, (cap + 255) / 256 + 1);
-    pack_facet_kernel<<<blocks, 256, 0, s>>>(dfacet, uu, vv, dre, dim, s2, pk, invs2, invs2_64,
-                                             cid, facet, dc, loff);
+    const unsigned blocks = std::min(2048u, (n + 255) / 256 + 1);
+    pack_facet_kernel<<<blocks, 256, 0, s>>>(n, uu, vv, dre, dim, s2, pk, invs2, invs2_64, dc);
 }
 
 // ------------------------------------------------------------------ r-marginalisation (K4)

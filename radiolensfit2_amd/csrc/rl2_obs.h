@@ -27,7 +27,7 @@ struct FacetSlot {
     uint32_t *loff = nullptr;// LDS record offsets per cell (fused Newton passes)
     double *ctr = nullptr;   // cell-centre coordinate per grid index (fmax)
     unsigned facet = 0;
-    unsigned n = 0;          // host copy of the compacted size (valid after a sync)
+    unsigned n = 0;          // host copy of the cell count (Obs::h_n after a sync)
     double rprior[kMaxR] = {};
 };
 
@@ -88,6 +88,10 @@ struct Obs {
     std::vector<FacetSlot> slots;
     FacetDev *d_facets = nullptr;
     std::vector<FacetDev> h_facets;
+    unsigned *h_n = nullptr;  // cell count per slot, written by compactions (pinned)
+    unsigned *d_n = nullptr;  // its device view
+    // cells and weights of the facet last extracted for a caller (pinned, small facets)
+    double *h_cells = nullptr, *d_cells = nullptr;
     LikBuffers lik;
     RGrid rg;
     int lik_block = 0;       // 0: tiled engine; 64..1024: one work-group per (item, r)
@@ -127,8 +131,11 @@ bool ensure_device();
 struct PendingSub {
     double l0, m0, flux, R_mu, e1, e2;
 };
+// What an extraction leaves besides the slot's facet: the dense weights in the slot's sumw, or
+// cells and weights in h_cells (facets up to host_cells only).
+enum class ExtractCopy { none, weights, host };
 bool obs_extract(Obs &o, int slot, double l0, double m0, double flux, double R_mu,
-                 unsigned facet, bool want_sumw, double e1 = 0., double e2 = 0.,
+                 unsigned facet, ExtractCopy copy, double e1 = 0., double e2 = 0.,
                  const PendingSub *sub = nullptr);
 bool obs_subtract(Obs &o, double l0, double m0, double flux, double R_mu, double e1, double e2);
 // One galaxy of a batched extraction into slot `slot`.

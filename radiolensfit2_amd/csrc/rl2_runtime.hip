@@ -299,6 +299,10 @@ Obs::~Obs()
         dfree(s.loff);
     }
     dfree(d_facets);
+    if (h_n) (void)hipHostFree(h_n);
+    if (h_cells) (void)hipHostFree(h_cells);
+    h_n = nullptr;
+    h_cells = nullptr;
     dfree(d_feat);
     for (auto &g : batch_graphs) (void)hipGraphExecDestroy(g.second);
     batch_graphs.clear();
@@ -337,6 +341,17 @@ bool Obs::ensure_slots(int n)
                     "memset"))
             return false;
     }
+    unsigned *hn = nullptr, *dn = nullptr;
+    if (!hip_ok(hipHostMalloc((void **)&hn, n * sizeof(unsigned)), "hipHostMalloc")) return false;
+    if (!hip_ok(hipHostGetDevicePointer((void **)&dn, hn, 0), "device view") ||
+        !hip_ok(hipStreamSynchronize(g_stream), "ensure_slots")) {  // compactions write h_n
+        (void)hipHostFree(hn);
+        return false;
+    }
+    for (int i = 0; i < n; i++) hn[i] = i < old && h_n ? h_n[i] : 0u;
+    if (h_n) (void)hipHostFree(h_n);
+    h_n = hn;
+    d_n = dn;
     FacetDev *nd = nullptr;
     if (!dmalloc(&nd, n)) return false;
     if (d_facets) {
@@ -381,11 +396,7 @@ bool Obs::facet_upload(int i)
 {
     FacetDev &f = h_facets[i];
     for (int k = 0; k < kMaxR; k++) f.rprior[k] = slots[i].rprior[k];
-    const size_t off = offsetof(FacetDev, rprior);
-    return hip_ok(hipMemcpyAsync((char *)(d_facets + i) + off, (char *)&f + off,
-                                 sizeof(FacetDev) - off, hipMemcpyHostToDevice, g_stream),
-                  "facet descriptor") &&
-           hip_ok(hipMemcpyAsync(d_facets + i, &f, offsetof(FacetDev, n), hipMemcpyHostToDevice,
+    return hip_ok(hipMemcpyAsync(d_facets + i, &f, offsetof(FacetDev, n), hipMemcpyHostToDevice,
                                  g_stream),
                   "facet descriptor");
 }
@@ -443,17 +454,64 @@ static bool ensure_stream2()
            hip_ok(hipEventCreateWithFlags(&g_join, hipEventDisableTiming), "hipEventCreate");
 }
 
+// Where a slot's compaction writes.
+static CompactOut compact_out(Obs &o, int slot)
+{
+    const FacetSlot &s = o.slots[slot];
+    CompactOut c = {};
+    c.uu = s.uu;
+    c.vv = s.vv;
+    c.dre = s.dre;
+    c.dim = s.dim;
+    c.s2 = s.s2;
+    c.n_out = &o.d_facets[slot].n;
+    c.cid = s.cid;
+    c.ctr = s.ctr;
+    c.pk = s.pk;
+    c.invs2 = s.invs2;
+    c.invs2_64 = s.invs2_64;
+    c.dc = s.dc;
+    c.loff = s.loff;
+    c.n_host = o.d_n + slot;
+    return c;
+}
+
+// A facet returned to a caller: up to this many grid cells the compaction writes the cells and
+// weights to pinned host memory itself.  Six copies to the caller's pageable arrays and one of
+// the count cost 85 us of the 169 us of a whole extraction into 1,024 grid cells, now 60; beyond
+// the limit (3 MB of pinned memory) the copies' bandwidth is what counts.
+constexpr size_t kHostCells = 65536;
+static size_t host_cells(const Obs &o)
+{
+    return std::min((size_t)o.fmax * o.fmax, kHostCells);
+}
+
 // Compaction of a slot's accumulators into its facet, the FP32 copy and the descriptor.
-static bool finish_extract(Obs &o, int slot, unsigned facet, bool want_sumw, const AccScale &sc)
+static bool finish_extract(Obs &o, int slot, unsigned facet, ExtractCopy copy, const AccScale &sc)
 {
     FacetSlot &s = o.slots[slot];
-    if (want_sumw && !s.sumw && !dmalloc(&s.sumw, (size_t)o.fmax * o.fmax)) return false;
+    CompactOut c = compact_out(o, slot);
+    const size_t cap = host_cells(o);
+    if (copy == ExtractCopy::host) {
+        if (!o.d_cells) {
+            if (!o.h_cells && !hip_ok(hipHostMalloc((void **)&o.h_cells, 6 * cap * sizeof(double)),
+                                      "hipHostMalloc"))
+                return false;
+            if (!hip_ok(hipHostGetDevicePointer((void **)&o.d_cells, o.h_cells, 0), "device view"))
+                return false;
+        }
+        c.h_vis = reinterpret_cast<double2 *>(o.d_cells);
+        c.h_s2 = o.d_cells + 2 * cap;
+        c.h_uu = o.d_cells + 3 * cap;
+        c.h_vv = o.d_cells + 4 * cap;
+        c.sum_w = o.d_cells + 5 * cap;
+    } else if (copy == ExtractCopy::weights) {
+        if (!s.sumw && !dmalloc(&s.sumw, (size_t)o.fmax * o.fmax)) return false;
+        c.sum_w = s.sumw;
+    }
     {
         KTimer t(RL2_K_COMPACT);
-        launch_compact(g_stream, s.acc, facet, o.len, s.uu, s.vv, s.dre, s.dim, s.s2, s.cid,
-                       s.ctr, &o.d_facets[slot].n, want_sumw ? s.sumw : nullptr, s.scan, &sc);
-        launch_pack_facet(g_stream, &o.d_facets[slot], facet * facet, s.uu, s.vv, s.dre, s.dim,
-                          s.s2, s.pk, s.invs2, s.invs2_64, s.cid, facet, s.dc, s.loff);
+        launch_compact(g_stream, s.acc, facet, o.len, c, s.scan, &sc);
     }
     // the facet now has grid structure: cell ids and centres for the phase tables (packed
     // in 16-bit row / column fields)
@@ -469,7 +527,7 @@ static bool finish_extract(Obs &o, int slot, unsigned facet, bool want_sumw, con
 }
 
 bool obs_extract(Obs &o, int slot, double l0, double m0, double flux, double R_mu,
-                 unsigned facet, bool want_sumw, double e1, double e2, const PendingSub *sub)
+                 unsigned facet, ExtractCopy copy, double e1, double e2, const PendingSub *sub)
 {
     if (facet == 0 || facet > o.fmax) {
         set_error("facet size " + std::to_string(facet) + " outside the allocated facet (max " +
@@ -518,7 +576,7 @@ bool obs_extract(Obs &o, int slot, double l0, double m0, double flux, double R_m
     stats_add_work(RL2_K_EXTRACT, 0., o.nvis * (bytes_per_vis(o, RL2_K_EXTRACT) +
                                                 (sub ? (o.prec == 0 ? 16. : 8.) : 0.)) +
                                           o.nrow * 24.);
-    return finish_extract(o, slot, facet, want_sumw, sc) &&
+    return finish_extract(o, slot, facet, copy, sc) &&
            hip_ok(hipGetLastError(), "extract launch");
 }
 
@@ -611,19 +669,7 @@ bool obs_extract_batch(Obs &o, const std::vector<ExtractReq> &reqs,
         Cp.acc = sl.acc;
         Cp.fx_unscale = 1.0 / sc.fx_scale;
         Cp.fs_unscale = 1.0 / sc.fs_scale;
-        Cp.uu = sl.uu;
-        Cp.vv = sl.vv;
-        Cp.dre = sl.dre;
-        Cp.dim = sl.dim;
-        Cp.s2 = sl.s2;
-        Cp.cid = sl.cid;
-        Cp.ctr = sl.ctr;
-        Cp.dc = sl.dc;
-        Cp.loff = sl.loff;
-        Cp.pk = sl.pk;
-        Cp.invs2 = sl.invs2;
-        Cp.invs2_64 = sl.invs2_64;
-        Cp.n_out = &o.d_facets[r.slot].n;
+        Cp.out = compact_out(o, r.slot);
         Cp.scan = sl.scan;
         Cp.facet = r.facet;
         Cp.pad = 0;
@@ -1115,9 +1161,9 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
 
 static bool read_slot_n(Obs &o, int slot, unsigned *n)
 {
-    return hip_ok(hipMemcpyAsync(n, &o.d_facets[slot].n, sizeof *n, hipMemcpyDeviceToHost, g_stream),
-                  "copy n") &&
-           hip_ok(hipStreamSynchronize(g_stream), "sync");
+    if (!hip_ok(hipStreamSynchronize(g_stream), "sync")) return false;
+    *n = o.h_n[slot];
+    return true;
 }
 
 static bool prior_for(Obs &o, int slot, double flux)
@@ -1282,8 +1328,8 @@ bool process_list(Obs &o, const std::vector<unsigned> &todo, int pass, const dou
             const unsigned gal = todo[b0 + k];
             if (!prior_for(o, (int)k, flux[gal])) return false;
             const unsigned facet = facet_size(scale[gal], o.len);
-            if (!obs_extract(o, (int)k, l[gal], m[gal], flux[gal], scale[gal], facet, false, 0.,
-                             0., pending ? &pend : nullptr))
+            if (!obs_extract(o, (int)k, l[gal], m[gal], flux[gal], scale[gal], facet,
+                             ExtractCopy::none, 0., 0., pending ? &pend : nullptr))
                 return false;
             pending = false;
             results[gal].facet = facet;
@@ -1668,12 +1714,30 @@ int rl2_obs_extract(rl2_obs *obs, int slot, double l0, double m0, double flux, d
 {
     if (!obs || slot < 0) return RL2_ERR_ARG;
     Obs &o = obs->o;
-    if (!obs_extract(o, slot, l0, m0, flux, R_mu, facet, sum_w != nullptr)) return RL2_ERR_HIP;
+    const bool host = (facet_vis || facet_sigma2 || uu || vv || sum_w) &&
+                      (size_t)facet * facet <= host_cells(o);
+    if (!obs_extract(o, slot, l0, m0, flux, R_mu, facet,
+                     host    ? ExtractCopy::host
+                     : sum_w ? ExtractCopy::weights
+                             : ExtractCopy::none))
+        return RL2_ERR_HIP;
     unsigned n = 0;
     if (!read_slot_n(o, slot, &n)) return RL2_ERR_HIP;
     FacetSlot &s = o.slots[slot];
     s.n = n;
     if (ncoords) *ncoords = n;
+    if (host) {
+        const size_t cap = host_cells(o);
+        auto take = [&](double *h, int array, size_t count) {
+            if (h) memcpy(h, o.h_cells + array * cap, count * sizeof(double));
+        };
+        take(facet_vis, 0, 2 * (size_t)n);
+        take(facet_sigma2, 2, n);
+        take(uu, 3, n);
+        take(vv, 4, n);
+        take(sum_w, 5, (size_t)facet * facet);
+        return RL2_OK;
+    }
     std::vector<double> re, im;
     auto down = [](void *h, const void *d, size_t bytes) {
         return hip_ok(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, g_stream), "extract copy");
@@ -1721,8 +1785,8 @@ int rl2_obs_load_facet(rl2_obs *obs, int slot, unsigned int n, const double *fac
               up(s.s2, facet_sigma2, n * 8) && up(s.uu, uu, n * 8) && up(s.vv, vv, n * 8) &&
               up(&o.d_facets[slot].n, &n, sizeof n);
     if (ok)
-        launch_pack_facet(g_stream, &o.d_facets[slot], n, s.uu, s.vv, s.dre, s.dim, s.s2, s.pk,
-                          s.invs2, s.invs2_64, nullptr, 0, s.dc, s.loff);
+        launch_pack_facet(g_stream, n, s.uu, s.vv, s.dre, s.dim, s.s2, s.pk, s.invs2,
+                          s.invs2_64, s.dc);
     FacetDev &f = o.h_facets[slot];  // caller-given cells: no grid structure
     if (ok && (f.cid || f.grid_facet)) {
         f.cid = nullptr;
@@ -1733,6 +1797,7 @@ int rl2_obs_load_facet(rl2_obs *obs, int slot, unsigned int n, const double *fac
     ok = hip_ok(hipStreamSynchronize(g_stream), "load_facet") && ok;  // before n and re, im go
     if (!ok) return RL2_ERR_HIP;
     s.n = n;
+    o.h_n[slot] = n;
     return RL2_OK;
 }
 

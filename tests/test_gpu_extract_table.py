@@ -14,10 +14,10 @@ pytestmark = pytest.mark.gpu
 LEN, NCH, FLUX, SCALE = 93000.0, 5, 80.0, 1.0
 
 
-def _observation(nrow, spread, special):
+def _observation(nrow, spread, special, length=LEN):
     rng = np.random.default_rng(nrow)
     wn = 2 * np.pi / np.linspace(0.25, 0.22, NCH)
-    r = {"one": 2.0, "wide": 0.2 * LEN}[spread]  # metres: a cell or two, or a cell per row
+    r = {"one": 2.0, "wide": 0.2 * length}[spread]  # metres: a cell or two, or a cell per row
     u, v = rng.uniform(-r, r, (2, nrow)) + 300.0
     n = nrow * NCH
     vis = rng.standard_normal(n) + 1j * rng.standard_normal(n)
@@ -28,7 +28,7 @@ def _observation(nrow, spread, special):
         vis[1] = complex(np.nan, 1.0)
         s2[nrow + 2] = np.nan
     spec = np.linspace(1.0, 0.9, NCH)
-    return synth.Observation(None, u, v, rng.uniform(-50, 50, nrow), wn, spec, s2, flag, LEN, vis)
+    return synth.Observation(None, u, v, rng.uniform(-50, 50, nrow), wn, spec, s2, flag, length, vis)
 
 
 @pytest.mark.parametrize("precision", [N.RL2_PREC_FP64, N.RL2_PREC_MIXED])
@@ -69,3 +69,29 @@ def test_extraction_table_matches_the_runs_and_the_oracle(gpu, nrow, spread, pre
         np.testing.assert_array_equal(got[2], want[2])
         np.testing.assert_array_equal(got[3], want[3])
         np.testing.assert_array_equal(got[4], want[4])
+
+
+@pytest.mark.parametrize("spread", ["one", "wide"])
+@pytest.mark.parametrize("facet", [1, 2, 31, 32, 33, 64, 97, 255, 256, 257, 300])
+def test_compaction_at_the_edges_of_its_tiles(gpu, facet, spread):
+    """Facets of less than, exactly and more than whole tiles of 1,024 cells, and either side of
+    the 65,536 cells whose copies the compaction writes for the caller, against the oracle."""
+    obs = _observation(3000, spread, False, 3 * LEN)  # facets of up to 360 columns
+    zero = np.zeros(obs.nvis, np.complex128)
+    gal = (2e-4, -1e-4, FLUX, SCALE)
+    dev = P.DeviceObservation(obs, vis_sky=zero)
+    try:
+        dev.extract(*gal, facet)
+        got = dev.extract(*gal, facet)  # on accumulators that a compaction has cleared
+        n = dev.extract_only(*gal, facet)
+    finally:
+        dev.close()
+    want = O.extract(obs, *gal, facet, obs.vis, zero)
+    assert n == len(got[0]) == len(want[0])
+    w = want[4][want[4] != 0]
+    top = FLUX + np.abs(obs.vis).max()
+    # as above; sums of up to 15,000 FP64 terms in the reference's order: 15,000 / 2 ulp at worst
+    assert (np.abs(got[0] - want[0]) / w).max() <= 1e-12 * top * 2
+    np.testing.assert_allclose(got[1], want[1], rtol=1e-12)
+    for k in (2, 3, 4):
+        np.testing.assert_array_equal(got[k], want[k])
