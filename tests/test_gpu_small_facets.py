@@ -72,3 +72,26 @@ def test_small_facets_match_the_passes_and_the_oracle(gpu, n, points):
             assert abs(got[0][k] - le) <= 1e-8
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("n", [200, 9000])
+@pytest.mark.parametrize("points", [1, 8, 9, 40])
+def test_results_polled_for_are_those_of_a_synchronised_evaluation(gpu, n, points):
+    """Evaluations that return on their results (L_e alone, L_r of up to 8 points) in turns on one
+    set of buffers, and one that synchronises (with statistics): the same bits every time."""
+    dev = _facet_of(n)[0]
+    try:
+        e = np.random.default_rng(points).uniform(-0.5, 0.5, (2, points, 2))
+        P.stats_enable(True)
+        want = [dev.loglik(x[:, 0], x[:, 1], detail=True) for x in e]
+        P.stats_enable(False)
+        for _ in range(3):
+            for x, w in zip(e, want):
+                for detail in (False, True):
+                    got = dev.loglik(x[:, 0], x[:, 1], detail=detail)
+                    for a, b in zip(got, w):
+                        np.testing.assert_array_equal(a[..., 1:] if a.ndim == 2 else a,
+                                                      b[..., 1:] if b.ndim == 2 else b)
+    finally:
+        P.stats_enable(False)
+        dev.close()
