@@ -213,7 +213,7 @@ int rl2_synchronize(void);
  *   tables of 512 / 1024 / 2048 / 1024 / 2048 slots, flushed to the facet after every
  *   channel; 6 runs of 4 rows with 2048 slots that keep their cells across channels and are
  *   flushed only when the next channel might not fit; 5 (default, the fastest) pairs of rows
- *   of 1,024-row blocks with several copies of each cell's sums (plain gridding, weights and
+ *   of 512-row blocks with several copies of each cell's sums (plain gridding, weights and
  *   visibilities without a finite bound: runs of 2 rows with 1024 slots, as 6).  Every
  *   variant accumulates in integers, so the facet does not depend on the order of the
  *   work-groups (variants with the same rows per work-group give the same bits).

@@ -430,26 +430,29 @@ __global__ __launch_bounds__(256) void grid_run_kernel(GridLaunch a)
     }
 }
 
-// ---- extraction's default: one LDS table per work-group with a copy of every sum per lane
+// ---- extraction's default: one LDS table per work-group with several copies of every sum
 // Sorted rows put a wave's visibilities of a channel into two to four cells (64 rows of a
 // 197-dish observation into 1.7 cells at 296 columns, 3.2 at 924), so a table with one sum per
 // cell made the LDS atomics of 64 lanes wait for each other on one address: they were half of
 // the extraction.  Here lane l adds to copy l % 4 of a cell's sums, which are in different
-// banks, and the copies are added when the table is flushed.  512 threads of 2 rows and 512
-// cells of 4 copies: 60 KB, two work-groups per CU, the 16 waves that 128 registers allow.  1,024
-// rows and all channels of that array have 30 to 190 cells.  74M visibilities (complex128, 8
-// channels) take 1.09 ms (runs merged in registers, one sum per cell: 1.41; with the subtraction
-// 1.48 against 1.62), 15M in complex64 0.27 ms (0.37), 0.8M in 16 channels 31 us (51; 43
-// against 58).  What is left is FP64 arithmetic (two thirds of the issue slots) and the LDS
-// atomics.  Fewer cells (256) take 3% longer where corners of the uv plane overflow, 2 copies
-// 4%, 1 row per thread or 3 waves per SIMD 25% to 30%; loading a channel ahead gives nothing.
+// banks, and the copies are added when the table is flushed.  256 threads of 2 rows and 256
+// cells of 4 copies: 30 KB, five work-groups per CU, the 20 waves that 100 registers allow (with
+// the subtraction 16); 512 rows and all channels of that array have 20 to 120 cells.
+// 148M visibilities (complex128, 16 channels) take 0.78 ms into 296 columns and 1.05 into 924
+// (runs merged in registers, one sum per cell: 1.42), 1.27 with the subtraction (1.62), 29M in
+// complex64 0.23 ms (0.37), 3.9M in 4 channels 27 us (51).  The bytes take 0.61 ms (1.09 with
+// the subtraction) at the rate of a large copy; what is left is FP64 arithmetic (over half of
+// the issue slots) and the LDS atomics.  512 threads and 512 cells take 0.92, 1.13, 1.32 and
+// 0.27 ms (16 waves, and a work-group's sparse rows keep more waves waiting), 128 threads 25%
+// more on the smallest, 128 cells 1% to 4%, 2 copies 4%, a row per thread 25%; runs kept in
+// registers across channels 9%; loading a channel ahead gives nothing.
 // A visibility that finds no place in kCellProbes steps goes to the accumulators directly, so
 // the table has no size that must suffice, and it is flushed when three quarters are in use
 // (looked at every four channels) and at the end.  The integer sums make the facet the same
 // bit for bit however the visibilities are spread over copies and flushes.
 // Values are rounded by adding 1.5 * 2^52 (|x| 2^S < 2^51 by fx_scales, which needs finite
 // bounds: the host takes the kernel above otherwise); a NaN counts as 0, as its conversion did.
-constexpr int kCellBS = 512, kCellRows = 2, kCellSlots = 512, kCellCopies = 4, kCellProbes = 8;
+constexpr int kCellBS = 256, kCellRows = 2, kCellSlots = 256, kCellCopies = 4, kCellProbes = 8;
 struct CellTable {
     unsigned long long sum[3][kCellSlots * kCellCopies];  // re, im, sigma^2
     uint32_t cnt[kCellSlots * kCellCopies];
@@ -478,8 +481,8 @@ __device__ inline void cell_clear(CellTable &T)
 __device__ inline void cell_add(CellTable &T, double *accd, unsigned long ncell, uint32_t key,
                                 long long re, long long im, long long s2, uint32_t n)
 {
-    uint32_t h = (key * 2654435761u) >> 23;
-    static_assert(kCellSlots == 1 << 9, "hash bits");
+    uint32_t h = (key * 2654435761u) >> 24;
+    static_assert(kCellSlots == 1 << 8, "hash bits");
 #pragma unroll 1
     for (int p = 0; p < kCellProbes; p++) {
         uint32_t k = __hip_atomic_load(&T.key[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -570,7 +573,7 @@ __device__ inline bool cell_term(CellTerm &o, const GridLaunch &a, double u_inc,
 
 // SUB: the previous galaxy's post-fit update in the same pass, as grid_run_kernel.
 template <int PREC, bool SUB>
-__global__ __launch_bounds__(kCellBS, 4) void grid_cell_kernel(GridLaunch a)
+__global__ __launch_bounds__(kCellBS, SUB ? 4 : 5) void grid_cell_kernel(GridLaunch a)
 {
     constexpr int RPT = kCellRows;
     static_assert(RPT == 2, "a pair of rows");

@@ -1,4 +1,4 @@
-"""The extraction's default gridding (one table of cells per 1,024 rows, several copies of each
+"""The extraction's default gridding (one table of cells per 512 rows, several copies of each
 sum): observations at the edges of its row blocks, in few cells and in more than its table holds,
 against the run-merging variant (bit for bit: integer sums of the same terms) and the oracle."""
 import numpy as np
@@ -33,7 +33,7 @@ def _observation(nrow, spread, special, length=LEN):
 
 @pytest.mark.parametrize("precision", [N.RL2_PREC_FP64, N.RL2_PREC_MIXED])
 @pytest.mark.parametrize("spread", ["one", "wide"])
-@pytest.mark.parametrize("nrow", [1, 2, 3, 1023, 1024, 1025, 2049, 5001])
+@pytest.mark.parametrize("nrow", [1, 2, 3, 511, 512, 513, 1023, 1024, 1025, 2049, 5001])
 def test_extraction_table_matches_the_runs_and_the_oracle(gpu, nrow, spread, precision):
     H = N.hip()
     facet = H.facet_size(SCALE, LEN)
