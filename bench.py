@@ -488,7 +488,7 @@ def roofline(kstats, lik_peak, fused=True):
     (lik_p0_group_kernel, or lik_tile_kernel, for pass 0, and lik_fused_kernel /
     lik_fused_wide_kernel for the Newton passes when the steps are folded into them, else
     lik_tile_kernel; FP64 VALU) and the extraction's gridding
-    kernel (grid_run_kernel, HBM).
+    kernel (grid_cell_kernel, HBM).
     achieved = the device-counted algorithmic FLOP-equivalents (bytes) of the timed launches
     / their summed durations from HIP events around each launch on the library stream."""
     lik, ext, step = kstats["likelihood"], kstats["extract"], kstats["step"]
@@ -506,7 +506,7 @@ def roofline(kstats, lik_peak, fused=True):
              "valu_busy": tr.get("likelihood_tile_valu_busy"),
              "step_kernel": {"launches": step["launches"],
                              "avg_launch_us": round(1e3 * step["ms"] / max(1, step["launches"]), 3)}}
-    r_ext = {"kernel": "grid_run_kernel (extraction)", "bound": "hbm",
+    r_ext = {"kernel": "grid_cell_kernel (extraction)", "bound": "hbm",
              "achieved": round(ext_gbs, 2),
              "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": round(ext_gbs / PEAK_HBM_GBS, 5),
              "traffic": tr.get("extraction_launch_bytes"), "launches": ext["launches"],

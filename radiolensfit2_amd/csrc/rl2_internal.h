@@ -157,7 +157,7 @@ struct GridLaunch {
     double *acc;               // grid_acc_words(facet) words
     double fx_scale = 1., fs_scale = 1.;  // AccScale of the launch
     bool finite = false;       // the bounds behind the scales are finite
-    // mode 0, gridding variant 3 only: apply this post-fit update to the residual first
+    // mode 0, gridding variants 3, 5 and 6: apply this post-fit update to the residual first
     // (written back through res_w), then grid the updated visibilities
     int sub = 0;
     GalaxyGeom sfit, srnd;

@@ -4037,7 +4037,8 @@ __global__ __launch_bounds__(kTileBS, kTileGridWaves) void lik_persist_kernel(Pe
 // and a launch of their own is a small part of the evaluation.
 // Measured against the passes: one point on 138 cells 64.1 -> 46.5 us, the loop over 24
 // galaxies of 175 to 2111 cells 38.5 -> 26.3 ms, in batches of 16 (48 galaxies) 18.4 -> 15.1
-// ms.  On 6,582 cells 1, 4 and 24 points took 69, 71 and 102 us by the passes and 60, 60 and
+// ms (32 us, 17 and 9 ms with the shorter chains, the integral folded in and the results polled
+// for).  On 6,582 cells 1, 4 and 24 points took 69, 71 and 102 us by the passes and 60, 60 and
 // 96 here; from 8,192 cells on (twice the cells in registers, which spill) 71, 77 and 128
 // against 75, 76 and 139, so kTaskChunks is 4.
 template <int KIND, int G, int NC>
