@@ -73,6 +73,18 @@ __device__ inline double model_shape_rsq(const GalaxyGeom &g, double u, double v
 {
     return model_shape_kk(g, model_kk(g, u, v), wn2, spectra);
 }
+// For any galaxy a caller may name: an ellipticity on the unit circle, or a scalelength without a
+// finite square, has an infinite denominator and the model 0 (as 1 / (den sqrt(den)) gives it),
+// where rsqrt_ge1's residual would be infinity times 0.  A NaN stays one (the estimate's).
+__device__ inline double model_shape_any(const GalaxyGeom &g, double u, double v, double wn2,
+                                         double spectra)
+{
+    const double a = fma(g.sf * wn2, model_kk(g, u, v), 1.);
+    const double r = __builtin_amdgcn_rsq(a);
+    const double e = fma(-fmin(a, 1.7976931348623157e308) * r, r, 1.);
+    const double rr = fma(r * e, fma(e, 0.375, 0.5), r);
+    return rr * rr * rr * (spectra * g.flux);
+}
 
 // One visibility of the post-fit update (data_processing.c:109-135): R = (R - fit) + round,
 // both models with the phase rotor of the fitted galaxy's position (p = u l + v m + w n,
@@ -133,7 +145,7 @@ __device__ inline void add_sources_block(const GalaxyGeom *__restrict__ gal, uns
             for (int k = 0; k < CB; k++) {
                 // the phase k p in revolutions is p / lambda
                 const double wnc = wn[c0 + k];
-                const double shape = model_shape_rsq(g, ui, vi, wnc * wnc, spec[c0 + k]);
+                const double shape = model_shape_any(g, ui, vi, wnc * wnc, spec[c0 + k]);
                 double sn, cs;
                 sincos_rev64(p * inv_lambda[c0 + k], sn, cs);
                 are[k] = fma(shape, cs, are[k]);
