@@ -74,16 +74,18 @@ __device__ inline double model_shape_rsq(const GalaxyGeom &g, double u, double v
     return model_shape_kk(g, model_kk(g, u, v), wn2, spectra);
 }
 // For any galaxy a caller may name: an ellipticity on the unit circle, or a scalelength without a
-// finite square, has an infinite denominator and the model 0 (as 1 / (den sqrt(den)) gives it),
-// where rsqrt_ge1's residual would be infinity times 0.  A NaN stays one (the estimate's).
+// finite square, has an infinite denominator a and the model 0 (as 1 / (a sqrt(a)) gives it); a
+// NaN stays one (the estimate's).  a^(-3/2) is formed from the hardware's estimate r directly,
+// r^3 (1 + 3/2 e + 15/8 e^2) with e = 1 - a r^2 to twice the precision: two roundings, where the
+// cube of a rounded reciprocal root carries three of the root's.
 __device__ inline double model_shape_any(const GalaxyGeom &g, double u, double v, double wn2,
                                          double spectra)
 {
     const double a = fma(g.sf * wn2, model_kk(g, u, v), 1.);
-    const double r = __builtin_amdgcn_rsq(a);
-    const double e = fma(-fmin(a, 1.7976931348623157e308) * r, r, 1.);
-    const double rr = fma(r * e, fma(e, 0.375, 0.5), r);
-    return rr * rr * rr * (spectra * g.flux);
+    const double r = __builtin_amdgcn_rsq(a), b = fmin(a, 1.7976931348623157e308);
+    const double h = r * r, hl = fma(r, r, -h), r3 = h * r;
+    const double e = fma(-b, hl, fma(-b, h, 1.));
+    return fma(r3 * e, fma(e, 1.875, 1.5), r3) * (spectra * g.flux);
 }
 
 // One visibility of the post-fit update (data_processing.c:109-135): R = (R - fit) + round,
@@ -113,12 +115,12 @@ __device__ inline double2 subtract_vis(const GalaxyGeom &fit, const GalaxyGeom &
 // ------------------------------------------------------------------ sources / noise
 // R += sign * sum_g flux_g spec_c shape_g exp(i k_c (u l + v m + w n)).
 // One thread per row; galaxies staged through LDS in tiles of 128.
-// Bound by FP64 issue (a phase and a model per galaxy and visibility, 55 FP64 and integer
-// instructions), so the phase goes through sincos_rev64 and the model through one reciprocal
+// Bound by FP64 issue (a phase and a model per galaxy and visibility, about 60 FP64 and integer
+// instructions), so the phase goes through sincos_rev_near and the model through one reciprocal
 // square root, and whole blocks of CB channels run without a test per channel.  500 galaxies
-// on 3.87M visibilities: 3.7 ms; 7.3 with the library's sincos and a square root and a division
-// per model (the error against 64 bits, 1.6e-12 of the model on phases of up to 100
-// revolutions, is the phase's own rounding in both).
+// on 3.87M visibilities: 3.4 ms; 6.1 with the library's sincos and a square root and a division
+// per model.  The error against 80 bits is 0.87 of that form's (2.0e-15 against 2.3e-15 of the
+// model, rms, on phases of up to 40 revolutions; 0.92 of it in the modulus).
 template <int PREC, int CB>
 __device__ inline void add_sources_block(const GalaxyGeom *__restrict__ gal, unsigned ngal,
                                          unsigned c0, unsigned long nrow, unsigned long i,
@@ -129,9 +131,16 @@ __device__ inline void add_sources_block(const GalaxyGeom *__restrict__ gal, uns
 {
     constexpr int TILE = 128;
     __shared__ GalaxyGeom sg[TILE];
-    double are[CB], aim[CB];
+    // what 1 / lambda lacks of k / (2 pi): the phase then carries no rounding but that of p, where
+    // the product k p carries its own (1 / lambda alone would add two)
+    constexpr double kTwoPiLo = 2.4492935982947064e-16;
+    double are[CB], aim[CB], il_lo[CB];
 #pragma unroll
-    for (int k = 0; k < CB; k++) are[k] = aim[k] = 0.;
+    for (int k = 0; k < CB; k++) {
+        are[k] = aim[k] = 0.;
+        const double il = inv_lambda[c0 + k];
+        il_lo[k] = (fma(-il, kTwoPi, wn[c0 + k]) - il * kTwoPiLo) * (1. / kTwoPi);
+    }
     for (unsigned g0 = 0; g0 < ngal; g0 += TILE) {
         __syncthreads();
         for (unsigned t = threadIdx.x; t < TILE && g0 + t < ngal; t += blockDim.x)
@@ -146,8 +155,9 @@ __device__ inline void add_sources_block(const GalaxyGeom *__restrict__ gal, uns
                 // the phase k p in revolutions is p / lambda
                 const double wnc = wn[c0 + k];
                 const double shape = model_shape_any(g, ui, vi, wnc * wnc, spec[c0 + k]);
+                const double il = inv_lambda[c0 + k], t = p * il;
                 double sn, cs;
-                sincos_rev64(p * inv_lambda[c0 + k], sn, cs);
+                sincos_rev_near((t - rint(t)) + fma(p, il_lo[k], fma(p, il, -t)), sn, cs);
                 are[k] = fma(shape, cs, are[k]);
                 aim[k] = fma(shape, sn, aim[k]);
             }

@@ -97,10 +97,10 @@ RL2_HD double fma_const(double a, double b, double c)
 // ever subtracted.  q is rounded by adding 1.5 * 2^52, which leaves it in the low bits of m,
 // and the quadrant is chosen without branches: 26 FP64 and 9 integer instructions, where
 // rint, a conversion and nested selections took 27 and 30 and split the wave.
-RL2_HD void sincos_rev64(double t, double &sn, double &cs)
+// sincos_rev_near takes r = t - rint(t) (|r| up to a little over 1/2).
+RL2_HD void sincos_rev_near(double r, double &sn, double &cs)
 {
     const double kRound = 6755399441055744.;
-    const double r = t - rint(t);
     const double m = fma(r, 4., kRound);
     const double q = m - kRound;
     const double y = fma(-0.25, q, r);
@@ -129,6 +129,10 @@ RL2_HD void sincos_rev64(double t, double &sn, double &cs)
     const double a = odd ? c : s, b = odd ? s : c;
     sn = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, a) ^ ((k & 2) << 62));
     cs = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, b) ^ (((k + 1) & 2) << 62));
+}
+RL2_HD void sincos_rev64(double t, double &sn, double &cs)
+{
+    sincos_rev_near(t - rint(t), sn, cs);
 }
 
 // cell_index (evaluate_uv_grid.c:166-178) with each quotient (u / lambda + len) / inc as one

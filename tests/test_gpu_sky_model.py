@@ -1,5 +1,5 @@
-"""The sky model's kernel (rl2_obs_add_sources) on what a catalog may hold at its limits, against
-the model's own expression in plain FP64."""
+"""The sky model's kernel (rl2_obs_add_sources): what a catalog may hold at its limits, and its
+accuracy, against the model's own expression in plain FP64 and in 80 bits."""
 import numpy as np
 import pytest
 
@@ -38,7 +38,8 @@ def _sum_of_models(obs, cat, real=np.float64):
             det = 1 - e1 * e1 - e2 * e2
             sf = (s * real(ARCSEC)) ** 2 / (det * det)
             kk = ((1 + e1) * u + e2 * v) ** 2 + (e2 * u + (1 - e1) * v) ** 2
-            p = u * l + v * m + w * (np.sqrt(1 - l * l - m * m) - 1)
+            n = real(np.sqrt(1 - cat.l[g] ** 2 - cat.m[g] ** 2) - 1)  # the host forms it, in FP64
+            p = u * l + v * m + w * n
             for c in range(obs.nch):
                 k = real(obs.wn[c])
                 den = 1 + sf * k * k * kk
@@ -78,3 +79,36 @@ def test_sources_at_the_limits_of_a_catalog(gpu, nch, precision):
             assert np.all(np.abs(got[ok] - want[ok]) <= tol * 80.), name
     finally:
         dev.close()
+
+
+def _rms(x):
+    return float(np.sqrt(np.mean(np.abs(x.astype(np.clongdouble)) ** 2)))
+
+
+@pytest.mark.parametrize("reach", [3e-4, 1e-2, 0.3])
+@pytest.mark.parametrize("metres", [5e3, 150e3])
+def test_sources_are_as_accurate_as_the_plain_expression(gpu, metres, reach):
+    """The error against 80 bits is no larger than that of the model's expression in FP64
+    (k p, cos, sin, 1 / (den sqrt(den))), in the whole value and in its modulus."""
+    rng = np.random.default_rng(int(metres))
+    obs = _empty_observation(*rng.uniform(-metres, metres, (2, 5000)),
+                             rng.uniform(-0.1, 0.1, 5000) * metres, 6)
+    dev = P.DeviceObservation(obs)
+    err, mod = [], []
+    try:
+        dev.checkpoint()
+        for g in range(8):
+            cat = _catalog([(50., rng.uniform(.3, 3.), *rng.uniform(-.4, .4, 2),
+                             *rng.uniform(-reach, reach, 2))])
+            dev.restore()
+            dev.add_sources(cat)
+            plain = _sum_of_models(obs, cat)
+            true = _sum_of_models(obs, cat, np.longdouble)
+            size = np.abs(true)
+            err.append([(x - true) / size for x in (dev.residual(), plain)])
+            mod.append([np.abs(x.astype(np.clongdouble)) / size - 1 for x in (dev.residual(), plain)])
+    finally:
+        dev.close()
+    for kind in (err, mod):
+        got, plain = (np.concatenate([x[k] for x in kind]) for k in (0, 1))
+        assert _rms(got) <= _rms(plain), (_rms(got), _rms(plain))
