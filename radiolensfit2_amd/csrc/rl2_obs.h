@@ -26,6 +26,11 @@ struct FacetSlot {
     double2 *dc = nullptr;   // packed {D_re, D_im} (fused Newton passes)
     uint32_t *loff = nullptr;// LDS record offsets per cell (fused Newton passes)
     double *ctr = nullptr;   // cell-centre coordinate per grid index (fmax)
+    // Cells and weights of the facet last extracted for a caller, in pinned memory with its
+    // device view (facets up to kHostCells): the slot's own, so that threads may extract into
+    // different slots.  Six arrays of cells_cap, grown to the largest facet asked for.
+    double *h_cells = nullptr, *d_cells = nullptr;
+    size_t cells_cap = 0;
     unsigned facet = 0;
     unsigned n = 0;          // host copy of the cell count (Obs::h_n after a sync)
     double rprior[kMaxR] = {};
@@ -90,8 +95,6 @@ struct Obs {
     std::vector<FacetDev> h_facets;
     unsigned *h_n = nullptr;  // cell count per slot, written by compactions (pinned)
     unsigned *d_n = nullptr;  // its device view
-    // cells and weights of the facet last extracted for a caller (pinned, small facets)
-    double *h_cells = nullptr, *d_cells = nullptr;
     LikBuffers lik;
     RGrid rg;
     int lik_block = 0;       // 0: tiled engine; 64..1024: one work-group per (item, r)
@@ -132,7 +135,7 @@ struct PendingSub {
     double l0, m0, flux, R_mu, e1, e2;
 };
 // What an extraction leaves besides the slot's facet: the dense weights in the slot's sumw, or
-// cells and weights in h_cells (facets up to host_cells only).
+// cells and weights in its h_cells (facets up to kHostCells only).
 enum class ExtractCopy { none, weights, host };
 bool obs_extract(Obs &o, int slot, double l0, double m0, double flux, double R_mu,
                  unsigned facet, ExtractCopy copy, double e1 = 0., double e2 = 0.,

@@ -300,12 +300,12 @@ Obs::~Obs()
         dfree(s.ctr);
         dfree(s.dc);
         dfree(s.loff);
+        if (s.h_cells) (void)hipHostFree(s.h_cells);
+        s.h_cells = nullptr;
     }
     dfree(d_facets);
     if (h_n) (void)hipHostFree(h_n);
-    if (h_cells) (void)hipHostFree(h_cells);
     h_n = nullptr;
-    h_cells = nullptr;
     dfree(d_feat);
     for (auto &g : batch_graphs) (void)hipGraphExecDestroy(g.second);
     batch_graphs.clear();
@@ -484,9 +484,19 @@ static CompactOut compact_out(Obs &o, int slot)
 // the count cost 85 us of the 169 us of a whole extraction into 1,024 grid cells, now 60; beyond
 // the limit (3 MB of pinned memory) the copies' bandwidth is what counts.
 constexpr size_t kHostCells = 65536;
-static size_t host_cells(const Obs &o)
+static bool ensure_host_cells(FacetSlot &s, size_t ncell)
 {
-    return std::min((size_t)o.fmax * o.fmax, kHostCells);
+    if (ncell <= s.cells_cap) return true;
+    if (s.h_cells) (void)hipHostFree(s.h_cells);  // read by the call that filled it
+    s.h_cells = s.d_cells = nullptr;
+    s.cells_cap = 0;
+    size_t cap = 1024;
+    while (cap < ncell) cap *= 2;
+    if (!hip_ok(hipHostMalloc((void **)&s.h_cells, 6 * cap * sizeof(double)), "hipHostMalloc") ||
+        !hip_ok(hipHostGetDevicePointer((void **)&s.d_cells, s.h_cells, 0), "device view"))
+        return false;
+    s.cells_cap = cap;
+    return true;
 }
 
 // Compaction of a slot's accumulators into its facet, the FP32 copy and the descriptor.
@@ -494,20 +504,13 @@ static bool finish_extract(Obs &o, int slot, unsigned facet, ExtractCopy copy, c
 {
     FacetSlot &s = o.slots[slot];
     CompactOut c = compact_out(o, slot);
-    const size_t cap = host_cells(o);
     if (copy == ExtractCopy::host) {
-        if (!o.d_cells) {
-            if (!o.h_cells && !hip_ok(hipHostMalloc((void **)&o.h_cells, 6 * cap * sizeof(double)),
-                                      "hipHostMalloc"))
-                return false;
-            if (!hip_ok(hipHostGetDevicePointer((void **)&o.d_cells, o.h_cells, 0), "device view"))
-                return false;
-        }
-        c.h_vis = reinterpret_cast<double2 *>(o.d_cells);
-        c.h_s2 = o.d_cells + 2 * cap;
-        c.h_uu = o.d_cells + 3 * cap;
-        c.h_vv = o.d_cells + 4 * cap;
-        c.sum_w = o.d_cells + 5 * cap;
+        if (!ensure_host_cells(s, (size_t)facet * facet)) return false;
+        c.h_vis = reinterpret_cast<double2 *>(s.d_cells);
+        c.h_s2 = s.d_cells + 2 * s.cells_cap;
+        c.h_uu = s.d_cells + 3 * s.cells_cap;
+        c.h_vv = s.d_cells + 4 * s.cells_cap;
+        c.sum_w = s.d_cells + 5 * s.cells_cap;
     } else if (copy == ExtractCopy::weights) {
         if (!s.sumw && !dmalloc(&s.sumw, (size_t)o.fmax * o.fmax)) return false;
         c.sum_w = s.sumw;
@@ -1802,7 +1805,7 @@ int rl2_obs_extract(rl2_obs *obs, int slot, double l0, double m0, double flux, d
     if (!obs || slot < 0) return RL2_ERR_ARG;
     Obs &o = obs->o;
     const bool host = (facet_vis || facet_sigma2 || uu || vv || sum_w) &&
-                      (size_t)facet * facet <= host_cells(o);
+                      (size_t)facet * facet <= kHostCells;
     if (!obs_extract(o, slot, l0, m0, flux, R_mu, facet,
                      host    ? ExtractCopy::host
                      : sum_w ? ExtractCopy::weights
@@ -1814,9 +1817,8 @@ int rl2_obs_extract(rl2_obs *obs, int slot, double l0, double m0, double flux, d
     s.n = n;
     if (ncoords) *ncoords = n;
     if (host) {
-        const size_t cap = host_cells(o);
         auto take = [&](double *h, int array, size_t count) {
-            if (h) memcpy(h, o.h_cells + array * cap, count * sizeof(double));
+            if (h) memcpy(h, s.h_cells + array * s.cells_cap, count * sizeof(double));
         };
         take(facet_vis, 0, 2 * (size_t)n);
         take(facet_sigma2, 2, n);
