@@ -101,6 +101,8 @@ inline void rgrid_factor(RGrid &g)
     g.factored = 1;
 }
 
+unsigned num_cus();  // of the library's device
+
 // Streaming-kernel arguments (one galaxy).
 struct GalaxyGeom {
     double l0, m0, n0;         // n0 = sqrt(1 - l^2 - m^2) - 1

@@ -594,8 +594,10 @@ __device__ inline bool cell_term(CellTerm &o, const GridLaunch &a, double u_inc,
 }
 
 // SUB: the previous galaxy's post-fit update in the same pass, as grid_run_kernel.
+// Each work-group takes its rows' channels from blockIdx.y * channels on.
 template <int PREC, bool SUB>
-__global__ __launch_bounds__(kCellBS, SUB ? 4 : 5) void grid_cell_kernel(GridLaunch a)
+__global__ __launch_bounds__(kCellBS, SUB ? 4 : 5) void grid_cell_kernel(GridLaunch a,
+                                                                         unsigned channels)
 {
     constexpr int RPT = kCellRows;
     static_assert(RPT == 2, "a pair of rows");
@@ -633,7 +635,8 @@ __global__ __launch_bounds__(kCellBS, SUB ? 4 : 5) void grid_cell_kernel(GridLau
         ps[k] = a.s2f + i;
     }
     __syncthreads();
-    for (unsigned c = 0; c < a.nch; c++) {
+    const unsigned c0 = blockIdx.y * channels, c1 = min(a.nch, c0 + channels);
+    for (unsigned c = c0; c < c1; c++) {
         const double wn = a.wn[c], inv_lambda = a.inv_lambda[c];
         const double wn2 = wn * wn, spectra = a.spec[c];
         // both rows' values together: each line is still there for the second load
@@ -684,7 +687,7 @@ __global__ __launch_bounds__(kCellBS, SUB ? 4 : 5) void grid_cell_kernel(GridLau
             more = first && in[1] && !pair;
             first = false;
         }
-        if ((c & 3) == 3 && c + 1 < a.nch) {
+        if ((c & 3) == 3 && c + 1 < c1) {
             __syncthreads();
             const uint32_t used = T.used;
             __syncthreads();  // every thread has read it before any adds a cell
@@ -700,12 +703,26 @@ static void launch_grid_variant(hipStream_t s, const GridLaunch &a)
 {
     if (MODE == 0 && tuning().grid_variant == 5 && a.finite &&
         !(a.sub && (a.g.e1 != 0. || a.g.e2 != 0. || a.srnd.e1 != 0. || a.srnd.e2 != 0.))) {
+        // A work-group goes through its channels one after the other, 3 to 5 us each, and with many
+        // of them its rows' cells outgrow the table (a cell moves with the wavelength).  So the
+        // channels are shared out: 16 at most to a work-group, and with few rows fewer, four at
+        // least, until the work-groups fill the chip twice (one wave of them ends with its
+        // slowest).  Merging runs / all channels in one work-group / shared out: 2,760 rows of 64
+        // channels into 134 columns 233 / 343 / 45 us, 20,160 of 256 into 142 columns 766 / 1,288 /
+        // 110, 201,600 of 64 into 82 columns 246 / 337 / 121, 714,000 of 128 into 1,110 columns
+        // 2.66 / 2.51 / 2.03 ms, 685,440 of 128 into 1,216 columns 3.39 / 3.61 / 2.80 ms.  Eight
+        // channels at most are 0 to 5% slower near the array's core and as much faster far from
+        // it; 32 up to 20% slower.
         constexpr unsigned rows = kCellRows * kCellBS;
-        const dim3 grid((unsigned)((a.nrow + rows - 1) / rows));
+        const unsigned blocks = (unsigned)((a.nrow + rows - 1) / rows);
+        const unsigned fill = 2 * (a.sub ? 4 : 5) * num_cus();
+        const unsigned shares = std::max({1u, fill / blocks, (a.nch + 15) / 16});
+        const unsigned channels = ((a.nch + shares - 1) / shares + 3) / 4 * 4;
+        const dim3 grid(blocks, (a.nch + channels - 1) / channels);
         if (a.sub)
-            grid_cell_kernel<PREC, true><<<grid, kCellBS, 0, s>>>(a);
+            grid_cell_kernel<PREC, true><<<grid, kCellBS, 0, s>>>(a, channels);
         else
-            grid_cell_kernel<PREC, false><<<grid, kCellBS, 0, s>>>(a);
+            grid_cell_kernel<PREC, false><<<grid, kCellBS, 0, s>>>(a, channels);
         return;
     }
     if (tuning().grid_variant == 5) {

@@ -587,7 +587,7 @@ bool obs_extract(Obs &o, int slot, double l0, double m0, double flux, double R_m
 }
 
 static unsigned g_num_cus = 0;
-static unsigned num_cus()
+unsigned num_cus()
 {
     if (!g_num_cus) {
         hipDeviceProp_t p;
