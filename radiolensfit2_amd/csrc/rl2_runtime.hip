@@ -180,13 +180,17 @@ bool LikBuffers::ensure(int n)
     ok = ok && hip_ok(hipMemsetAsync(d_tasks, 0, (size_t)c * kMaxR * 2 * sizeof(TileTask),
                                      g_stream),
                       "memset");
-    // the results block lives in pinned host memory that the kernels write directly: the
-    // host reads it after the evaluation's one synchronisation, with no copy launch
-    ok = ok && hip_ok(hipHostMalloc((void **)&h_out, ob), "hipHostMalloc") &&
+    // The results (and L_r and the step counts on request) live in pinned host memory that the
+    // kernels write directly, with no copy launch.  Coherent by request, whatever the default is:
+    // the host polls these words while the launches run (Arrivals).
+    constexpr unsigned kCoherent = hipHostMallocCoherent;
+    ok = ok && hip_ok(hipHostMalloc((void **)&h_out, ob, kCoherent), "hipHostMalloc") &&
          hip_ok(hipHostGetDevicePointer((void **)&d_out, h_out, 0), "hipHostGetDevicePointer") &&
          hip_ok(hipHostMalloc((void **)&h_items, c * sizeof(LikItem)), "hipHostMalloc") &&
-         hip_ok(hipHostMalloc((void **)&h_Lr, (size_t)c * kMaxR * sizeof(double)), "hipHostMalloc") &&
-         hip_ok(hipHostMalloc((void **)&h_nit, (size_t)c * kMaxR * sizeof(int)), "hipHostMalloc") &&
+         hip_ok(hipHostMalloc((void **)&h_Lr, (size_t)c * kMaxR * sizeof(double), kCoherent),
+                "hipHostMalloc") &&
+         hip_ok(hipHostMalloc((void **)&h_nit, (size_t)c * kMaxR * sizeof(int), kCoherent),
+                "hipHostMalloc") &&
          hip_ok(hipHostGetDevicePointer((void **)&d_Lr_host, h_Lr, 0), "hipHostGetDevicePointer") &&
          hip_ok(hipHostGetDevicePointer((void **)&d_nit_host, h_nit, 0), "hipHostGetDevicePointer");
     if (!ok) return false;
