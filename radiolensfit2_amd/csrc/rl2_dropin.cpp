@@ -611,8 +611,6 @@ int cross_correlation(unsigned long int n_uv_coords, double *grid_u, double *gri
         a.nit = b.d_nit;
         a.Le = b.d_Le;
         a.err = b.d_err;
-        a.qag_ws = b.d_ws;
-        a.qag_iws = b.d_iws;
         a.block = 256;
         a.ho = dho.p;
         a.det = ddet.p;

@@ -287,8 +287,6 @@ struct LikLaunch {
     int *nit;                  // nitems * kMaxR
     double *Le;                // nitems
     int *err;                  // nitems
-    double *qag_ws;            // nitems * kQagDoubles
-    int *qag_iws;              // nitems * kQagInts
     int block;                 // threads per work-group (64..1024)
     int prec;
     double *ho = nullptr;      // optional nitems * kMaxR: cross-correlation peak value

@@ -49,8 +49,6 @@ struct LikBuffers {
     double *d_flops = nullptr, *h_flops = nullptr;
     double *d_Le = nullptr, *h_Le = nullptr;
     int *d_err = nullptr, *h_err = nullptr;
-    double *d_ws = nullptr;
-    int *d_iws = nullptr;
     // tiled engine
     TileTask *d_tasks = nullptr;                         // cap * kMaxR
     double *d_partials = nullptr;

@@ -169,17 +169,20 @@ bool LikBuffers::ensure(int n)
     release();
     int c = 256;
     while (c < n) c *= 2;
+    // two generations of task state, then the counters: one allocation and one fill, since an
+    // observation's first evaluation pays for each: one allocation and fill more took about 40 us of it
+    const size_t tasks = (size_t)c * kMaxR * 2, counters = (size_t)c * kMaxR + kInlItems;
+    char *zeroed = nullptr;
     const size_t ob = 16 + 12 * (size_t)c;  // status[2] u32, FLOPs f64, L_e[c] f64, err[c] i32
     bool ok = dmalloc(&d_items, c) && dmalloc(&d_Lr, (size_t)c * kMaxR) &&
               dmalloc(&d_nit, (size_t)c * kMaxR) &&
-              dmalloc(&d_ws, (size_t)c * kQagDoubles) && dmalloc(&d_iws, (size_t)c * kQagInts) &&
-              dmalloc(&d_tasks, (size_t)c * kMaxR * 2) &&  // two generations of task state
-              dmalloc(&d_cnt, (size_t)c * kMaxR) && dmalloc(&d_arrived, kInlItems);
-    ok = ok && hip_ok(hipMemsetAsync(d_arrived, 0, kInlItems * sizeof(unsigned), g_stream),
-                      "memset");
-    ok = ok && hip_ok(hipMemsetAsync(d_tasks, 0, (size_t)c * kMaxR * 2 * sizeof(TileTask),
-                                     g_stream),
-                      "memset");
+              dmalloc(&zeroed, tasks * sizeof(TileTask) + counters * sizeof(unsigned)) &&
+              hip_ok(hipMemsetAsync(zeroed, 0, tasks * sizeof(TileTask) + counters * sizeof(unsigned),
+                                    g_stream),
+                     "memset");
+    d_tasks = reinterpret_cast<TileTask *>(zeroed);
+    d_cnt = zeroed ? reinterpret_cast<unsigned *>(d_tasks + tasks) : nullptr;
+    d_arrived = zeroed ? d_cnt + (size_t)c * kMaxR : nullptr;
     // The results (and L_r and the step counts on request) live in pinned host memory that the
     // kernels write directly, with no copy launch.  Coherent by request, whatever the default is:
     // the host polls these words while the launches run (Arrivals).
@@ -211,11 +214,8 @@ void LikBuffers::release()
     dfree(d_Lr);
     dfree(d_nit);
     d_out = nullptr;  // device view of h_out
-    dfree(d_ws);
-    dfree(d_iws);
-    dfree(d_tasks);
-    dfree(d_cnt);
-    dfree(d_arrived);
+    dfree(d_tasks);  // and the counters behind it
+    d_cnt = d_arrived = nullptr;
     d_Lr_host = nullptr;
     d_nit_host = nullptr;
     if (h_out) (void)hipHostFree(h_out);
@@ -879,8 +879,6 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
     a.nit = b.d_nit;
     a.Le = b.d_Le;
     a.err = b.d_err;
-    a.qag_ws = b.d_ws;
-    a.qag_iws = b.d_iws;
     a.block = o.lik_block;
     a.prec = o.prec;
     std::vector<int> hp(n);
