@@ -169,8 +169,8 @@ bool LikBuffers::ensure(int n)
     release();
     int c = 256;
     while (c < n) c *= 2;
-    // two generations of task state, then the counters: one allocation and one fill, since an
-    // observation's first evaluation pays for each: one allocation and fill more took about 40 us of it
+    // Two generations of task state, then the counters: one allocation and one fill, since an
+    // observation's first evaluation pays for each (one more of both took about 40 us of it).
     const size_t tasks = (size_t)c * kMaxR * 2, counters = (size_t)c * kMaxR + kInlItems;
     char *zeroed = nullptr;
     const size_t ob = 16 + 12 * (size_t)c;  // status[2] u32, FLOPs f64, L_e[c] f64, err[c] i32
@@ -953,7 +953,6 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
             min_chunks = min_chunks && chunk == kTileMinCells;
         }
         const unsigned total = chunks * (unsigned)nr;
-        if (!b.ensure_partials(2 * (size_t)total)) return false;  // two generations
         // one chunk count for every item (the points of one galaxy): the kernels then find a
         // work-group's item by a division instead of a search
         unsigned item_chunks = n > 0 ? chunks / (unsigned)n : 0u;
@@ -976,16 +975,26 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
         // offsets are 32-bit, and a work-group stages one task's column table (24 bytes per
         // column) in LDS: beyond either limit the passes evaluate sin/cos per cell
         if (ntab > 0xffffffffu || tab_facet * 24u > kTileLdsBytes) ntab = 0;
-        if (ntab && !b.ensure_tab(ntab)) return false;
+        // the scalelength tasks in one or two groups: the second group's passes run on a
+        // second stream, so one group's step kernels and launch gaps overlap the other's sums
+        const int ng = (tuning().tile_streams == 2 && nr >= 2 && ensure_stream2()) ? 2 : 1;
+        const bool tab_y_lds =
+            ntab && tuning().phase_tables == 2 && tab_facet * 40u <= kTileLdsBytes;
+        // Small facets: every pass of a task in one work-group, one launch per evaluation,
+        // with the same bits as the passes.  A knob that shapes the passes keeps them.
+        const bool one_launch = tuning().fuse_step == 1 && ng == 1 && tab_y_lds &&
+                                ntab_items == n && min_chunks && most_chunks <= kTaskChunks &&
+                                !tuning().tile_passes && !tuning().tile_blocks &&
+                                !tuning().tile_cells && tuning().p0_tasks == Tuning().p0_tasks;
+        // two generations of sums, and the tables: such an evaluation has neither
+        if (!one_launch && !b.ensure_partials(2 * (size_t)total)) return false;
+        if (!one_launch && ntab && !b.ensure_tab(ntab)) return false;
         if (n > kInlItems)  // few items travel with the first kernel's arguments instead
             q_ok = hip_ok(hipMemcpyAsync(b.d_items, b.h_items, n * sizeof(LikItem),
                                          hipMemcpyHostToDevice, g_stream),
                           "items copy") &&
                    q_ok;
         a.tasks = b.d_tasks;
-        // the scalelength tasks in one or two groups: the second group's passes run on a
-        // second stream, so one group's step kernels and launch gaps overlap the other's sums
-        const int ng = (tuning().tile_streams == 2 && nr >= 2 && ensure_stream2()) ? 2 : 1;
         TileLaunch tg[2];
         for (int g = 0; g < ng; g++) {
             TileLaunch &t = tg[g];
@@ -997,7 +1006,7 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
             t.partials = b.d_partials + (g == 0 ? 0 : (size_t)tg[0].nwg * 8);
             t.tab = ntab ? b.d_tab : nullptr;
             t.tab_lds_facet = ntab ? tab_facet : 0;
-            t.tab_y_lds = ntab && tuning().phase_tables == 2 && tab_facet * 40u <= kTileLdsBytes;
+            t.tab_y_lds = tab_y_lds;
             // the grid kernels when every item has tables (FP64 on an extracted facet); 2:
             // with the items in the kernel arguments
             t.grid = (ntab && ntab_items == n) ? (n <= kInlItems ? 2u : 1u) : 0u;
@@ -1112,11 +1121,7 @@ bool lik_eval(Obs &o, const std::vector<LikItem> &items, double *Le, int *err, d
                 return true;
             }
         }
-        // Small facets: every pass of a task in one work-group, one launch per evaluation,
-        // with the same bits as the passes.  A knob that shapes the passes keeps them.
-        if (fused && tuning().fuse_step == 1 && tg[0].tab_y_lds && min_chunks &&
-            most_chunks <= kTaskChunks && !tuning().tile_passes && !tuning().tile_blocks &&
-            !tuning().tile_cells && tuning().p0_tasks == Tuning().p0_tasks) {
+        if (one_launch) {
             if (g_stats_on) want_detail(true);  // the step counts for the FLOPs
             a.tasks = nullptr;                  // every task ends in the launch
             TileLaunch t = tg[0];
