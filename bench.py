@@ -207,14 +207,40 @@ def run_variants(dev, obs, cat, n_gal, opts, res_plain, plain_value):
     return out
 
 
-def measured_traffic():
-    """HBM bytes per launch from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE passes over
-    this workload (each counter scaled by what it reads for a copy of known size)."""
+def measured_traffic(config, kernels):
+    """Counters of `kernels` from the committed rocprofv3 passes over the workload `config` (HBM
+    bytes per launch, each counter scaled by what it reads for a copy of known size, and the
+    share of issue slots with a vector instruction), or {} where they were measured on other
+    kernels or another workload."""
     try:
         with open(os.path.join(ROOT, "profiles", "traffic.json")) as f:
-            return json.load(f)
+            recorded = json.load(f)
     except (OSError, ValueError):
         return {}
+    if recorded.get("config") != config:
+        return {}
+    for entry in recorded["measured"]:
+        if entry["kernels"] == kernels:
+            return entry
+    return {}
+
+
+def timed_kernels(args):
+    """The kernels whose launches the likelihood and the extraction timers hold."""
+    if args.lik_block:
+        lik = ["likelihood_kernel"]
+    elif args.lik_precision or not args.fuse_step:
+        lik = ["lik_tile_kernel"]
+    elif args.fuse_step == 2:
+        lik = ["lik_p0_group_kernel", "lik_persist_kernel"]
+    elif args.config == "64dish" and not (args.tile_cells or args.tile_passes or args.tile_blocks
+                                          or args.tile_streams == 2):
+        lik = ["lik_task_kernel"]
+    else:
+        lik = ["lik_p0_group_kernel", "lik_fused_kernel", "lik_fused_wide_kernel"]
+    if args.batch > 1:
+        return lik, ["grid_batch_kernel"]
+    return lik, ["grid_cell_kernel" if args.grid_variant == 5 else "grid_run_kernel"]
 
 
 def run_compare(ngal=100, batch=16, log_prefix="[compare]"):
@@ -483,33 +509,41 @@ def run_config1(ngal=100):
             "bad_fits": {"first_pass": st.n_bad_first, "after_refit": st.n_bad_final}}
 
 
-def roofline(kstats, lik_peak, fused=True):
-    """Rooflines of the two kernels that bound a galaxy: the likelihood's chunk-sum kernels
-    (lik_p0_group_kernel, or lik_tile_kernel, for pass 0, and lik_fused_kernel /
-    lik_fused_wide_kernel for the Newton passes when the steps are folded into them, else
-    lik_tile_kernel; FP64 VALU) and the extraction's gridding
-    kernel (grid_cell_kernel, HBM).
+LIK_WORK = {
+    "lik_task_kernel": "every pass of a task in one work-group, facets of up to 8,192 cells; with up "
+                       "to 8 points also the integral over the scalelength",
+    "lik_p0_group_kernel": "chunk sums of the zero-offset pass",
+    "lik_fused_kernel": "a Newton pass and the step before it",
+    "lik_fused_wide_kernel": "the same, facets of over 1,024 columns",
+    "lik_persist_kernel": "every Newton pass of an evaluation",
+    "lik_tile_kernel": "chunk sums of the zero-offset and Newton passes",
+    "likelihood_kernel": "a task's search in one work-group",
+}
+
+
+def roofline(kstats, lik_peak, args):
+    """Rooflines of the kernels that bound a galaxy: the likelihood's (FP64 VALU) and the
+    extraction's gridding (HBM), those that run with these options (timed_kernels).
     achieved = the device-counted algorithmic FLOP-equivalents (bytes) of the timed launches
     / their summed durations from HIP events around each launch on the library stream."""
     lik, ext, step = kstats["likelihood"], kstats["extract"], kstats["step"]
-    tr = measured_traffic()
+    lik_kernels, ext_kernels = timed_kernels(args)
+    lik_tr = measured_traffic(args.config, lik_kernels)
+    ext_tr = measured_traffic(args.config, ext_kernels)
     lik_tf = lik["flops"] / (lik["ms"] * 1e-3) / 1e12 if lik["ms"] > 0 else 0.0
     ext_gbs = ext["bytes"] / (ext["ms"] * 1e-3) / 1e9 if ext["ms"] > 0 else 0.0
-    r_lik = {"kernel": ("lik_p0_group_kernel + lik_fused_kernel / lik_fused_wide_kernel (chunk "
-                        "sums of the zero-offset and Newton passes, each Newton pass taking the "
-                        "previous step)" if fused
-                        else "lik_tile_kernel (chunk sums of the zero-offset and Newton passes)"),
+    r_lik = {"kernel": " + ".join(f"{k} ({LIK_WORK[k]})" for k in lik_kernels),
              "bound": "valu", "achieved": round(lik_tf, 4),
              "peak": lik_peak, "unit": "TFLOP/s", "frac": round(lik_tf / lik_peak, 5),
-             "traffic": tr.get("likelihood_tile_launch_bytes"), "launches": lik["launches"],
+             "traffic": lik_tr.get("launch_bytes"), "launches": lik["launches"],
              "avg_launch_us": round(1e3 * lik["ms"] / max(1, lik["launches"]), 3),
-             "valu_busy": tr.get("likelihood_tile_valu_busy"),
+             "valu_busy": lik_tr.get("valu_busy"),
              "step_kernel": {"launches": step["launches"],
                              "avg_launch_us": round(1e3 * step["ms"] / max(1, step["launches"]), 3)}}
-    r_ext = {"kernel": "grid_cell_kernel (extraction)", "bound": "hbm",
+    r_ext = {"kernel": " + ".join(ext_kernels) + " (extraction)", "bound": "hbm",
              "achieved": round(ext_gbs, 2),
              "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": round(ext_gbs / PEAK_HBM_GBS, 5),
-             "traffic": tr.get("extraction_launch_bytes"), "launches": ext["launches"],
+             "traffic": ext_tr.get("launch_bytes"), "launches": ext["launches"],
              "avg_launch_us": round(1e3 * ext["ms"] / max(1, ext["launches"]), 3)}
     return (r_lik if lik["ms"] >= ext["ms"] else r_ext), r_lik, r_ext
 
@@ -546,8 +580,8 @@ def main():
     ap.add_argument("--grid-variant", type=int, default=5, choices=[0, 1, 2, 3, 4, 5, 6],
                     help="extraction gridding: runs of 2 / 2 / 8 / 4 / 4 rows per thread with "
                          "tables of 512 / 1024 / 2048 / 1024 / 2048 slots flushed per channel "
-                         "(0-4), or runs of 2 / 4 rows with 1024 / 2048 slots kept across "
-                         "channels (5, 6)")
+                         "(0-4), pairs of rows with several copies of each cell's sums (5), or "
+                         "runs of 4 rows with 2048 slots kept across channels (6)")
     ap.add_argument("--phase-tables", type=int, default=2, choices=[0, 1, 2],
                     help="FP64 Newton phases from per-pass column x row tables with the rows "
                          "in LDS (2) or in global memory (1), or a sin/cos per cell (0)")
@@ -655,7 +689,7 @@ def main():
         log(f"[bench]   {k:10s} {s['ms']:10.2f} ms  {s['launches']:7d} launches")
     mixed = args.lik_precision != 0 or res_prec != N.RL2_PREC_FP64
     peak = PEAK_FP64_TFLOPS if args.lik_precision == 0 else PEAK_FP32_TFLOPS
-    dominant, r_lik, r_ext = roofline(kstats, peak, fused=bool(args.fuse_step))
+    dominant, r_lik, r_ext = roofline(kstats, peak, args)
 
     accept = None
     if args.compare_fp64:
