@@ -104,3 +104,28 @@ def test_many_channels_are_not_slower_than_merging_runs(gpu, dishes, times, nch,
     finally:
         dev.close()
     assert best[5] <= best[1], best
+
+
+@pytest.mark.parametrize("precision", [N.RL2_PREC_FP64, N.RL2_PREC_MIXED])
+@pytest.mark.parametrize("what", ["visibility", "sigma2", "flux"])
+def test_without_a_finite_bound_every_visibility_is_counted(gpu, what, precision):
+    """An infinite value leaves the integer sums without a scale: the run-merging kernel takes the
+    call, whichever variant is chosen.  Cells and weights are those of the data all the same."""
+    obs = _observation(1025, 5)
+    gal = (2e-4, -1e-4, 80.0, 1.0)
+    facet = N.hip().facet_size(1.0, LEN)
+    obs.flag[777] = False
+    dev = P.DeviceObservation(obs, precision=precision)
+    want = dev.extract(*gal, facet)
+    dev.close()
+    if what == "visibility":
+        obs.vis[777] = complex(-np.inf, 1.0)
+    elif what == "sigma2":
+        obs.sigma2[777] = np.inf
+    else:
+        gal = (2e-4, -1e-4, np.inf, 1.0)
+    dev = P.DeviceObservation(obs, precision=precision)
+    got = dev.extract(*gal, facet)
+    dev.close()
+    for k in (2, 3, 4):
+        np.testing.assert_array_equal(got[k], want[k])
