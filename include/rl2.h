@@ -196,7 +196,9 @@ typedef struct {
     double bytes;         /* algorithmic HBM bytes (streaming kernels) */
 } rl2_kernel_stat;
 /* RL2_K_LIKELIHOOD: the likelihood's chunk-sum kernels (pass 0 and the Newton passes, which
- * take the previous pass's step when steps are fused); RL2_K_STEP: the per-task step kernels
+ * take the previous pass's step when steps are fused); on extracted facets of up to 8,192
+ * cells the one kernel of an evaluation, which for up to 8 points also integrates over the
+ * scalelength (nothing is then under RL2_K_RMARG); RL2_K_STEP: the per-task step kernels
  * (after every pass with RL2_TUNE_FUSE_STEP 0, else once after an evaluation's last pass). */
 enum { RL2_K_EXTRACT = 0, RL2_K_COMPACT = 1, RL2_K_LIKELIHOOD = 2, RL2_K_RMARG = 3,
        RL2_K_SUBTRACT = 4, RL2_K_SOURCES = 5, RL2_K_STEP = 6, RL2_K_COUNT = 7 };
@@ -213,10 +215,10 @@ int rl2_synchronize(void);
  *   tables of 512 / 1024 / 2048 / 1024 / 2048 slots, flushed to the facet after every
  *   channel; 6 runs of 4 rows with 2048 slots that keep their cells across channels and are
  *   flushed only when the next channel might not fit; 5 (default, the fastest) pairs of rows
- *   of 512-row blocks with several copies of each cell's sums (plain gridding, weights and
- *   visibilities without a finite bound: runs of 2 rows with 1024 slots, as 6).  Every
- *   variant accumulates in integers, so the facet does not depend on the order of the
- *   work-groups (variants with the same rows per work-group give the same bits).
+ *   of blocks of 512 rows and at most 16 channels with several copies of each cell's sums
+ *   (plain gridding, weights and visibilities without a finite bound: runs of 2 rows with
+ *   1024 slots, as 6).  Every variant accumulates in integers of one scale, so the facet
+ *   does not depend on the variant or the order of the work-groups.
  * RL2_TUNE_TILE_CELLS: facet cells per work-group of the tiled likelihood, a power of two
  *   in [256, 65536], or 0 (default) to choose per launch (2048 to 65536).
  * RL2_TUNE_PHASE_TABLES: 2 (default) evaluates the FP64 Newton phases on extracted facets

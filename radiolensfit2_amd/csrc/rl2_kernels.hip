@@ -1609,7 +1609,7 @@ __device__ __attribute__((always_inline)) inline void finish_lr(const LikLaunch 
     __hip_atomic_store(a.Lr + (size_t)item * kMaxR + r, L, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
     a.nit[(size_t)item * kMaxR + r] = iter;
-    if (a.Lr_host) {  // pinned memory: the caller reads them after its one synchronisation
+    if (a.Lr_host) {  // pinned memory, where the host polls for them or reads them at the end
         a.Lr_host[(size_t)item * kMaxR + r] = L;
         a.nit_host[(size_t)item * kMaxR + r] = iter;
     }

@@ -50,13 +50,13 @@ struct LikBuffers {
     double *d_Le = nullptr, *h_Le = nullptr;
     int *d_err = nullptr, *h_err = nullptr;
     // tiled engine
-    TileTask *d_tasks = nullptr;                         // cap * kMaxR
+    TileTask *d_tasks = nullptr;                         // 2 * cap * kMaxR, then the counters
     double *d_partials = nullptr;
     size_t partials_cap = 0;                             // work-groups
     double *d_ppart = nullptr;                           // one-launch evaluations: chunk
     size_t ppart_cap = 0;                                // sums per pass (work-groups)
-    unsigned *d_cnt = nullptr;                           // cap * kMaxR chunk counters
-    unsigned *d_arrived = nullptr;                       // kInlItems task counters
+    unsigned *d_cnt = nullptr;                           // cap * kMaxR chunk counters, and
+    unsigned *d_arrived = nullptr;                       // kInlItems task counters: in d_tasks
     double *d_Lr_host = nullptr;                         // device views of h_Lr, h_nit
     int *d_nit_host = nullptr;
     double2 *d_tab = nullptr;                            // Newton phase tables
