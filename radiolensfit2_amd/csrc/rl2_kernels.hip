@@ -716,7 +716,8 @@ static void launch_grid_variant(hipStream_t s, const GridLaunch &a)
         constexpr unsigned rows = kCellRows * kCellBS;
         const unsigned blocks = (unsigned)((a.nrow + rows - 1) / rows);
         const unsigned fill = 2 * (a.sub ? 4 : 5) * num_cus();
-        const unsigned shares = std::max({1u, fill / blocks, (a.nch + 15) / 16});
+        const unsigned shares =  // (65,535 at most: the launch's limit)
+            std::min(65535u, std::max({1u, fill / blocks, (a.nch + 15) / 16}));
         const unsigned channels = ((a.nch + shares - 1) / shares + 3) / 4 * 4;
         const dim3 grid(blocks, (a.nch + channels - 1) / channels);
         if (a.sub)

@@ -590,16 +590,15 @@ bool obs_extract(Obs &o, int slot, double l0, double m0, double flux, double R_m
            hip_ok(hipGetLastError(), "extract launch");
 }
 
-static unsigned g_num_cus = 0;
 unsigned num_cus()
 {
-    if (!g_num_cus) {
+    static const unsigned n = [] {  // once, also for threads that extract at the same time
         hipDeviceProp_t p;
-        g_num_cus = hipGetDeviceProperties(&p, g_device) == hipSuccess && p.multiProcessorCount > 0
-                        ? (unsigned)p.multiProcessorCount
-                        : 256u;
-    }
-    return g_num_cus;
+        return hipGetDeviceProperties(&p, g_device) == hipSuccess && p.multiProcessorCount > 0
+                   ? (unsigned)p.multiProcessorCount
+                   : 256u;
+    }();
+    return n;
 }
 
 static bool ensure_batch_buffers(Obs &o)

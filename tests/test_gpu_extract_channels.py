@@ -6,6 +6,7 @@ import time
 import numpy as np
 import pytest
 
+from oracle import oracle as O
 from radiolensfit2_amd import _native as N
 from radiolensfit2_amd import pipeline as P
 from radiolensfit2_amd import synth
@@ -129,3 +130,23 @@ def test_without_a_finite_bound_every_visibility_is_counted(gpu, what, precision
     dev.close()
     for k in (2, 3, 4):
         np.testing.assert_array_equal(got[k], want[k])
+
+
+def test_more_channels_than_a_launch_has_shares_of_sixteen(gpu):
+    """1,048,577 channels are one more than 65,535 work-groups of sixteen; against the oracle."""
+    nch, nrow = 65535 * 16 + 17, 2
+    obs = _observation(nrow, nch)
+    facet = N.hip().facet_size(1.0, LEN)
+    gal = (2e-4, -1e-4, 80.0, 1.0)
+    zero = np.zeros(obs.nvis, np.complex128)
+    dev = P.DeviceObservation(obs, vis_sky=zero)
+    got = dev.extract(*gal, facet)
+    dev.close()
+    want = O.extract(obs, *gal, facet, obs.vis, zero)
+    for k in (2, 3, 4):
+        np.testing.assert_array_equal(got[k], want[k])
+    # a term is rounded to 2^-31 of the bound (1,024 rows of so many channels fit 62 bits), and
+    # a facet's visibility is sum(x) w / sum(sigma^2) over w terms, sigma^2 at least 0.5
+    w = want[4][want[4] != 0]
+    bound = 80.0 + 2 * np.abs(obs.vis).max()
+    assert (np.abs(got[0] - want[0]) / w).max() <= 2.0 ** -29 * bound
