@@ -1,6 +1,6 @@
 """Two host threads that extract into different slots of one observation, or evaluate on one each,
-get their own results: of an extraction the
-facet's cells, on facets whose cells the compaction writes for the caller and on wider ones."""
+get their own results (an extraction's cells on facets whose cells the compaction writes for the
+caller, and on wider ones)."""
 import threading
 
 import numpy as np
